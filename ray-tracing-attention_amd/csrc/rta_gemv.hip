@@ -1023,14 +1023,12 @@ int64_t rta_pack_bytes(int fmt, int rows, int cols) {
 static int pack_rows(int fmt, const void* src, int rows, int cols, const Remap& m, void* dst, hipStream_t s) {
     if (!dst) return RTA_ERR_NULL;
     if (reinterpret_cast<uintptr_t>(dst) % 16) return RTA_ERR_ALIGN;
-    const int64_t n2 = rta_pack_bytes(fmt, rows, cols) / 2;
-    const dim3 g((unsigned)((n2 + 255) / 256)), b(256);
+    const dim3 g((unsigned)((rows + 15) / 16), (unsigned)((cols / 256 + kPackSb - 1) / kPackSb)), b(256);
+    const uint8_t* from = static_cast<const uint8_t*>(src);
     if (fmt == RTA_Q4_K)
-        hipLaunchKernelGGL(pack_kernel<RTA_Q4_K>, g, b, 0, s, static_cast<const uint8_t*>(src), rows, cols,
-                           static_cast<uint8_t*>(dst), n2, m);
+        hipLaunchKernelGGL(pack_kernel<RTA_Q4_K>, g, b, 0, s, from, rows, cols, static_cast<uint8_t*>(dst), m);
     else
-        hipLaunchKernelGGL(pack_kernel<RTA_Q6_K>, g, b, 0, s, static_cast<const uint8_t*>(src), rows, cols,
-                           static_cast<uint8_t*>(dst), n2, m);
+        hipLaunchKernelGGL(pack_kernel<RTA_Q6_K>, g, b, 0, s, from, rows, cols, static_cast<uint8_t*>(dst), m);
     return hipGetLastError() == hipSuccess ? RTA_OK : RTA_ERR_LAUNCH;
 }
 
