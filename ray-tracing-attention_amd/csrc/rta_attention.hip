@@ -355,13 +355,20 @@ __device__ __forceinline__ void attn_plan_wave(const AttnArgs& a) {
         const int t = tiles_of(s);
         int before, total;
         scan(t, before, total);
-        if (s < a.nseq) {
-            const int64_t first = carry + before, end = first + t;
-            a.plan[s] = (int32_t)first;
-            if (T > 0 && t > 0) {
-                for (int64_t w = (first * P + T - 1) / T; w < (end * P + T - 1) / T && w < P; ++w)
-                    a.plan[a.nseq + 1 + w] = s;
-            }
+        if (s < a.nseq) a.plan[s] = (int32_t)(carry + before);
+        // The run of workgroups whose first tile lies in each sequence, written by the whole
+        // wave sequence by sequence (one lane writing its own sequence's run took 16 us for one
+        // sequence of 512 workgroups, and takes 4.7 so, launch included)
+        const int64_t first = carry + before, end = first + t;
+        int w0 = 0, w1 = 0;   // at most nwg workgroups
+        if (t > 0) {
+            w0 = (int)((first * P + T - 1) / T);
+            w1 = (int)((end * P + T - 1) / T);
+        }
+        const int here = a.nseq - s0 < kWave ? a.nseq - s0 : kWave;
+        for (int i = 0; i < here; ++i) {   // uniform
+            const int wb = __builtin_amdgcn_readlane(w1, i);
+            for (int w = __builtin_amdgcn_readlane(w0, i) + lane; w < wb; w += kWave) a.plan[a.nseq + 1 + w] = s0 + i;
         }
         carry += total;
     }
@@ -2051,27 +2058,31 @@ __global__ void __launch_bounds__(256) full_middle_kernel(const MiddleArgs p) {
     if (b == 0 && wave == 0 && p.plan.plan) attn_plan_wave(p.plan);
 }
 
-// One workgroup per (sequence, query head): 8 chunk groups x 32 lanes of 4
-// coordinates; every thread keeps 8 chunk records in flight.  One pass: each group
-// folds its records into a running (m, Z, U), rescaled when m grows, and the groups
-// are combined at the end (the same sums as max-then-accumulate, in another order).
-// GROUPS groups of 32 threads, kAhead records in flight per group: 16 (512 threads) when
-// a sequence's records can number in the hundreds (few sequences share the grid), else 8.
-template <int GROUPS>
-__global__ void __launch_bounds__(32 * GROUPS) attn_merge_kernel(const AttnArgs a) {
-    constexpr int kGroups = GROUPS, kAhead = 8;
-    __shared__ float4 s_u[kGroups][kHd / 4];
-    __shared__ float s_zp[kGroups], s_mp[kGroups];
-    const int sh = blockIdx.x;
+// Combines a sequence's chunk records per query head.  A workgroup owns 128 / SPLIT of a
+// head's coordinates: groups of 32 / SPLIT threads (4 coordinates each), kAhead records in
+// flight per group.  One pass: each group folds its records into a running (m, Z, U),
+// rescaled when m grows; the groups are combined inside each wave, then across the waves
+// (the same sums as max-then-accumulate, in another order).
+// Bound by latency: a handful of dependent reads of records another kernel just wrote.
+// With few (sequence, head) pairs the records per pair run to the hundreds and most compute
+// units would idle, so 512 threads take a quarter of the head each (64 records at once per
+// round of kAhead); see merge_split for the sizes.
+template <int THREADS, int SPLIT>
+__global__ void __launch_bounds__(THREADS) attn_merge_kernel(const AttnArgs a) {
+    constexpr int kLanes = 32 / SPLIT, kGroups = THREADS / kLanes, kAhead = 8;
+    constexpr int kWaves = THREADS / kWave, kCols = kHd / SPLIT;
+    __shared__ float4 s_u[kWaves][kLanes];
+    __shared__ float s_zp[kWaves], s_mp[kWaves];
+    const int sh = blockIdx.x / SPLIT, part = blockIdx.x - sh * SPLIT;
     const int s = sh / a.hq, h = sh - s * a.hq;
     const int tid = threadIdx.x;
-    const int grp = tid >> 5, e = tid & 31;
+    const int grp = tid / kLanes, e = part * kLanes + tid % kLanes;
     const int64_t L = a.ctx_len[s];
     const int64_t visible = L < a.capacity ? L : a.capacity;
     float* out = a.out + (int64_t)sh * kHd;
     if (visible <= 0) {
-        if (tid < kHd) out[tid] = 0.0f;
-        if (tid == 0) {
+        if (tid < kCols) out[part * kCols + tid] = 0.0f;
+        if (tid == 0 && part == 0) {
             if (a.m_out) a.m_out[sh] = -INFINITY;
             if (a.z_out) a.z_out[sh] = 0.0f;
             raise_error(RTA_DEVERR_HITS);
@@ -2140,31 +2151,48 @@ __global__ void __launch_bounds__(32 * GROUPS) attn_merge_kernel(const AttnArgs 
             }
         }
     }
-    s_u[grp][e] = U;
-    if (e == 0) {
-        s_zp[grp] = Z;
-        s_mp[grp] = Mg;
+    // combine the groups of a wave (every lane ends with its wave's sums)
+#pragma unroll
+    for (int off = kLanes; off < kWave; off <<= 1) {
+        const float M2 = __shfl_xor(Mg, off, kWave), Z2 = __shfl_xor(Z, off, kWave);
+        const float4 U2 = make_float4(__shfl_xor(U.x, off, kWave), __shfl_xor(U.y, off, kWave),
+                                      __shfl_xor(U.z, off, kWave), __shfl_xor(U.w, off, kWave));
+        const float M = fmaxf(Mg, M2);
+        const float f = Mg == -INFINITY ? 0.0f : expf(Mg - M), f2 = M2 == -INFINITY ? 0.0f : expf(M2 - M);
+        Z = fmaf(Z, f, Z2 * f2);
+        U.x = fmaf(U.x, f, U2.x * f2);
+        U.y = fmaf(U.y, f, U2.y * f2);
+        U.z = fmaf(U.z, f, U2.z * f2);
+        U.w = fmaf(U.w, f, U2.w * f2);
+        Mg = M;
+    }
+    const int wave = tid >> 6;
+    if ((tid & 63) < kLanes) s_u[wave][tid & 63] = U;
+    if ((tid & 63) == 0) {
+        s_zp[wave] = Z;
+        s_mp[wave] = Mg;
     }
     __syncthreads();
-    if (tid < kHd) {
+    if (tid < kCols) {
+        const int c = part * kCols + tid;   // coordinate of the head
         float M = -INFINITY;
 #pragma unroll
-        for (int g = 0; g < kGroups; ++g) M = fmaxf(M, s_mp[g]);
+        for (int g = 0; g < kWaves; ++g) M = fmaxf(M, s_mp[g]);
         float u = 0.0f, z = 0.0f;
 #pragma unroll
-        for (int g = 0; g < kGroups; ++g) {
+        for (int g = 0; g < kWaves; ++g) {
             const float f = s_mp[g] == -INFINITY ? 0.0f : expf(s_mp[g] - M);
             u = fmaf(reinterpret_cast<const float*>(&s_u[g][0])[tid], f, u);
             z = fmaf(s_zp[g], f, z);
         }
         float o = u / fmaxf(z, 1e-30f);
-        if (a.gate) o *= detector_sigmoid(a.gate[(int64_t)(sh / a.hq) * a.gate_stride + (sh % a.hq) * kHd + tid]);
+        if (a.gate) o *= detector_sigmoid(a.gate[(int64_t)s * a.gate_stride + h * kHd + c]);
         // with out_rotary R the head's rotary-pair order goes back to the exporter's
         // half-split column order (originalRotaryAxis), the columns the O projection's
         // axis remap reads (resident_quant.glsl:20,25)
         const int R = a.out_rotary;
-        out[tid < R ? (tid & 1) * (R >> 1) + (tid >> 1) : tid] = o;
-        if (tid == 0) {
+        out[c < R ? (c & 1) * (R >> 1) + (c >> 1) : c] = o;
+        if (c == 0) {
             if (a.m_out) a.m_out[sh] = M;
             if (a.z_out) a.z_out[sh] = z;
             if (short_grid) raise_error(RTA_DEVERR_HITS);
@@ -2672,8 +2700,15 @@ int decode_attention_gate_stride(const float* q, int nseq, int hq, int hkv, int 
     else if (fmt_k == RTA_Q6_K && fmt_v == RTA_Q4_K) e = launch_chunks<RTA_Q6_K, RTA_Q4_K>(G, a, lds, s);
     else e = launch_chunks<RTA_Q4_K, RTA_Q4_K>(G, a, lds, s);
     if (e != hipSuccess) return RTA_ERR_LAUNCH;
-    if (nseq <= 16) hipLaunchKernelGGL((attn_merge_kernel<16>), dim3(nseq * hq), dim3(512), 0, s, a);
-    else hipLaunchKernelGGL((attn_merge_kernel<8>), dim3(nseq * hq), dim3(256), 0, s, a);
+    // A sequence's records number up to min(its tiles, workgroups), split between the few
+    // sequences of a call.  Up to 128 of them are one round of 16 groups x 8 records, and from
+    // 65 (sequence, head) pairs on the pairs fill the chip by themselves: a quarter of a head
+    // per workgroup is then slower (16 x 16 pairs of ~190 records 45.6 -> 47.9 us per
+    // attention call, 32 pairs of ~60 records +0.7 us); 32 pairs of 512 records 16.5 -> 8.5 us
+    if (nseq * hq <= 64 && a.max_tiles > 128)
+        hipLaunchKernelGGL((attn_merge_kernel<512, 4>), dim3(nseq * hq * 4), dim3(512), 0, s, a);
+    else if (nseq <= 16) hipLaunchKernelGGL((attn_merge_kernel<512, 1>), dim3(nseq * hq), dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((attn_merge_kernel<256, 1>), dim3(nseq * hq), dim3(256), 0, s, a);
     return hipGetLastError() == hipSuccess ? RTA_OK : RTA_ERR_LAUNCH;
 }
 
