@@ -487,10 +487,11 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_mfma_kernel(
 
 // Adds the K-slab partials in slab order and applies the epilogue.  In kSwiglu the
 // virtual rows interleave gate (even) and up (odd).  kLogits also writes per-block
-// maxima pmax[b * gridDim.x + block] for the argmax.
+// maxima pmax[b * gridDim.x + block] for the argmax.  A slab holds slab_batch rows.
 template <int MODE, int NS>
 __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float* __restrict__ part, int nslab, int rows,
-                                                          int batch, float* __restrict__ y, float* __restrict__ pmax) {
+                                                          int batch, float* __restrict__ y, float* __restrict__ pmax,
+                                                          int slab_batch) {
     const int total_rows = MODE == kSwiglu ? 2 * rows : rows;
     const int b = blockIdx.y;
     const int r = blockIdx.x * 256 + threadIdx.x;
@@ -499,7 +500,7 @@ __global__ void __launch_bounds__(256) gemm_reduce_kernel(const float* __restric
         // every slab's value is loaded before the first add (see add_slabs)
         float s = 0.0f, s2 = 0.0f;
         const float* p0 = part + (int64_t)b * total_rows;
-        const int64_t ks = (int64_t)kMaxBatchTile * total_rows;
+        const int64_t ks = (int64_t)slab_batch * total_rows;
         if constexpr (NS == 0) {
             for (int k = 0; k < nslab; ++k) {
                 if constexpr (MODE == kSwiglu) {

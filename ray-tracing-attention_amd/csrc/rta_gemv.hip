@@ -5,6 +5,7 @@
 #include <climits>
 #include "rta_gemm.hpp"
 #include "rta_packed.hpp"
+#include "rta_wide.hpp"
 #include "rta_remap.hpp"
 #include "rta_gemv.hpp"
 #include "rta_host.hpp"
@@ -372,9 +373,9 @@ static MmaPlan plan_tiled(int rows, int cols, int nbt, bool dual) {
     return p;
 }
 
-// Bytes of workspace one projection needs (0 when the VALU paths serve it); covers
-// batch tiles of either width.
-static size_t projection_ws(int fmt, int rows, int cols, int batch, bool dual) {
+// Bytes of workspace one projection needs for its batch tiles of at most 32 rows (0 when
+// the VALU paths serve it); covers batch tiles of either width.
+static size_t narrow_ws(int fmt, int rows, int cols, int batch, bool dual) {
     if (is_tiled(fmt)) {
         const MmaPlan a = plan_tiled(rows, cols, 1, dual), b = plan_tiled(rows, cols, 2, dual);
         return a.x_bytes + (a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes);
@@ -384,14 +385,79 @@ static size_t projection_ws(int fmt, int rows, int cols, int batch, bool dual) {
     return a.x_bytes + (a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes);
 }
 
+// Work split of wide_kernel (rta_wide.hpp) for a call of `batch` rows in launches of up to
+// kWideBatch: the tile width and K slabs with the least estimated time.  One workgroup per
+// compute unit at a time; per superblock 17 MFMAs x 2 waves per SIMD for each of its TN x NB
+// tiles, a start of a few microseconds, and for K slabs the partials' trip through memory
+// and the reduce.  The plan follows the batch's class (64, 128, more) and not the batch, so
+// that a row's result does not depend on the rows beside it; up to 64 rows take the narrow
+// tiles' slabs (see kWideSplit).
+constexpr double kWideStartUs = 4.0, kWideTileUs = 0.2267, kWideReduceUs = 3.0, kWidePartUs = 2e-6;
+struct WidePlan {
+    int nb, tn, nslab, sb_per_slab, nblk;
+};
+
+static WidePlan plan_wide(int rows, int cols, int batch, bool dual) {
+    WidePlan best{};
+    const int most = batch <= 64 ? 64 : batch <= 128 ? 128 : kWideBatch;
+    const int ntile = (rows + 15) / 16, nsbt = cols / 256, nb = most > 64 ? 2 : 1;
+    const int mblk = most / (64 * nb);
+    const int narrow = nb == 1 ? plan_tiled(rows, cols, 2, dual).nslab : 0;
+    const double total = 16.0 * ntile * (dual ? 2 : 1);
+    double least = 0.0;
+    for (int tn = 4; tn <= 8; tn += 2) {
+        if (nb == 1 && tn == 6) continue;   // not built: the narrow batch block is bound by its start
+        const int per = dual ? tn : 2 * tn, nblk = (ntile + per - 1) / per;
+        for (int ns = 1; ns <= nsbt; ++ns) {
+            const int spb = (nsbt + ns - 1) / ns;
+            if ((nsbt + spb - 1) / spb != ns || (narrow && ns != narrow)) continue;
+            const int64_t rounds = ((int64_t)nblk * mblk * ns + kPlanCUs - 1) / kPlanCUs;
+            const double t = (double)rounds * (kWideStartUs + spb * tn * nb * kWideTileUs) +
+                             (ns > 1 ? kWideReduceUs + ns * most * total * kWidePartUs : 0.0);
+            if (best.tn == 0 || t < least) {
+                least = t;
+                best = WidePlan{nb, tn, ns, spb, nblk};
+            }
+        }
+    }
+    return best;
+}
+
+static bool wide_format(int fmt) { return is_tiled(fmt) || is_kquant(fmt); }
+
+static int one_tile(int batch) { return batch < kMaxBatchTile ? batch : kMaxBatchTile; }
+
+// x fragments, group sums and 1 / s of n rows
+static size_t wide_x_bytes(int cols, int n) {
+    const size_t b = (size_t)((n + 15) / 16) * (cols / 256) * (16384 + 1024 + 64);
+    return (b + 255) & ~(size_t)255;
+}
+
+// Workspace of the wide launches of a call of `batch` rows (0: it makes none).  GGUF rows up
+// to 64 stay on the narrow tiles, whose order of summation over K is another.
+static size_t wide_ws(int fmt, int rows, int cols, int batch, bool dual) {
+    if (!wide_format(fmt) || batch <= (is_tiled(fmt) ? kMaxBatchTile : 64)) return 0;
+    const WidePlan p = plan_wide(rows, cols, batch, dual);
+    const int n = batch < kWideBatch ? batch : kWideBatch;
+    return wide_x_bytes(cols, n) +
+           (p.nslab > 1 ? (size_t)p.nslab * n * (dual ? 2 : 1) * rows * sizeof(float) : 0);
+}
+
+// Workspace of a projection over `batch` rows: the narrow tiles' or the wide launches',
+// whichever is more (a caller may run a smaller batch on it).
+static size_t projection_ws(int fmt, int rows, int cols, int batch, bool dual) {
+    const size_t a = narrow_ws(fmt, rows, cols, one_tile(batch), dual), b = wide_ws(fmt, rows, cols, batch, dual);
+    return a > b ? a : b;
+}
+
 // The fixed-order slab reduce (gemm_reduce_kernel), its loads all in flight at once for
 // up to 16 slabs.
 template <int MODE>
 static void launch_reduce(dim3 grid, const float* part, int nslab, int rows, int batch, float* y, float* pmax,
-                          hipStream_t s) {
+                          hipStream_t s, int slab_batch = kMaxBatchTile) {
     with_slab_count(nslab, [&](auto ns) {
         hipLaunchKernelGGL((gemm_reduce_kernel<MODE, decltype(ns)::value>), grid, dim3(256), 0, s, part, nslab, rows,
-                           batch, y, pmax);
+                           batch, y, pmax, slab_batch);
     });
 }
 
@@ -468,6 +534,76 @@ static hipError_t run_tiled(int fmt, const Launch& l, void* ws, float* pmax, int
     return hipGetLastError();
 }
 
+template <int FMT, bool DUAL>
+static void launch_wide(const WidePlan& p, const WideArgs& a, hipStream_t s) {
+    const dim3 g(p.nblk, (a.batch + 64 * p.nb - 1) / (64 * p.nb), p.nslab), b(kWideThreads);
+    if (p.nb == 1) {
+        if (p.tn == 4) hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 1, 4>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 1, 8>), g, b, 0, s, a);
+    } else {
+        if (p.tn == 4) hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 2, 4>), g, b, 0, s, a);
+        else if (p.tn == 6) hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 2, 6>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 2, 8>), g, b, 0, s, a);
+    }
+}
+
+template <int FMT>
+static void launch_wide_xprep(const WidePlan& p, const float* x, int cols, int batch, const WideX& to, hipStream_t s) {
+    const dim3 g(cols / 256, (batch + 15) / 16), b(512);
+    if (kWideSplit<2> && p.nb == 2) hipLaunchKernelGGL((wide_xprep_kernel<FMT, true>), g, b, 0, s, x, cols, batch, to);
+    else hipLaunchKernelGGL((wide_xprep_kernel<FMT, false>), g, b, 0, s, x, cols, batch, to);
+}
+
+// Up to kWideBatch rows of a call with plan p: x fragments -> wide_kernel (-> fixed-order
+// slab reduce).
+template <int MODE>
+static hipError_t run_wide(int fmt, const WidePlan& p, const Launch& l, void* ws, float* pmax, int* ntasks_out,
+                           int* rpt_out, hipStream_t s) {
+    constexpr bool kDual = MODE == kSwiglu;
+    const int nsbt = l.cols / 256, rt = (l.batch + 15) / 16;
+    uint8_t* base = static_cast<uint8_t*>(ws);
+    WideArgs a{};
+    a.w = l.w;
+    a.w2 = l.w2;
+    a.row_bytes = l.row_bytes;
+    a.rows = l.rows;
+    a.nsbt = nsbt;
+    a.x.frag = reinterpret_cast<uint4*>(base);
+    a.x.g = a.x.frag + (size_t)rt * nsbt * 1024;
+    a.x.inv = reinterpret_cast<float*>(a.x.g + (size_t)rt * nsbt * 64);
+    a.batch = l.batch;
+    a.rt = rt;
+    a.y = l.y;
+    a.part = reinterpret_cast<float*>(base + wide_x_bytes(l.cols, l.batch));
+    a.pmax = pmax;
+    a.sb_per_slab = p.sb_per_slab;
+    a.mode = MODE;
+    if ((fmt & 0xff) == RTA_Q4_K) {
+        launch_wide_xprep<RTA_Q4_K>(p, l.x, l.cols, l.batch, a.x, s);
+        launch_wide<RTA_Q4_K, kDual>(p, a, s);
+    } else {
+        launch_wide_xprep<RTA_Q6_K>(p, l.x, l.cols, l.batch, a.x, s);
+        launch_wide<RTA_Q6_K, kDual>(p, a, s);
+    }
+    if (p.nslab > 1) {
+        const dim3 rg((l.rows + 255) / 256, l.batch);
+        launch_reduce<MODE>(rg, a.part, p.nslab, l.rows, l.batch, l.y, pmax, s, l.batch);
+        if (ntasks_out) *ntasks_out = (int)rg.x;
+        if (rpt_out) *rpt_out = 256;
+    } else {
+        if (ntasks_out) *ntasks_out = (l.rows + 15) / 16;
+        if (rpt_out) *rpt_out = 16;
+    }
+    return hipGetLastError();
+}
+
+// Whether a call of `batch` rows runs as wide launches: where the caller's workspace holds
+// them (one sized for a smaller batch leaves it to the narrow tiles).
+static bool use_wide(int fmt, int rows, int cols, int batch, bool dual, const void* ws, size_t ws_bytes) {
+    const size_t need = wide_ws(fmt, rows, cols, batch, dual);
+    return need && ws && ws_bytes >= need;
+}
+
 // Runs one projection over the whole batch: K-quant tiles of >= 8 rows on the matrix
 // cores (32 rows per tile), smaller ones on the VALU kernels (8 rows per tile).
 // For kLogits, partial receives per-task maxima laid out [tile row][ntasks] inside the
@@ -486,8 +622,10 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
     // depends on tiling.
     const bool mma = is_kquant(fmt) &&
                      mma_batch((int64_t)rows * cols * (MODE == kSwiglu ? 2 : 1), path_batch > 0 ? path_batch : batch);
+    const int whole = path_batch > 0 ? path_batch : batch;
+    const bool wide = !rn.part && use_wide(fmt, rows, cols, whole, MODE == kSwiglu, ws, ws_bytes);
     while (b0 < batch) {
-        const int cap = (mma || tiled) ? kMaxBatchTile : 8;
+        const int cap = wide ? kWideBatch : (mma || tiled) ? kMaxBatchTile : 8;
         const int chunk = batch - b0 < cap ? batch - b0 : cap;
         Launch l{};
         l.w = static_cast<const uint8_t*>(w);
@@ -503,11 +641,14 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
         if (rn.part) l.rn.part = rn.part + b0;
         l.xn = xn;
         hipError_t e;
-        if (tiled) {
-            if (!ws || ws_bytes < projection_ws(fmt, rows, cols, chunk, MODE == kSwiglu)) return RTA_ERR_WORKSPACE;
+        if (wide) {
+            e = run_wide<MODE>(fmt, plan_wide(rows, cols, whole, MODE == kSwiglu), l, ws, l.partial, ntasks_out,
+                               rows_per_task_out, s);
+        } else if (tiled) {
+            if (!ws || ws_bytes < narrow_ws(fmt, rows, cols, chunk, MODE == kSwiglu)) return RTA_ERR_WORKSPACE;
             e = run_tiled<MODE>(fmt, l, ws, l.partial, ntasks_out, rows_per_task_out, s);
         } else if (mma) {
-            if (!ws || ws_bytes < projection_ws(fmt, rows, cols, chunk, MODE == kSwiglu)) return RTA_ERR_WORKSPACE;
+            if (!ws || ws_bytes < narrow_ws(fmt, rows, cols, chunk, MODE == kSwiglu)) return RTA_ERR_WORKSPACE;
             e = run_mfma<MODE>(fmt, l, ws, l.partial, ntasks_out, rows_per_task_out, s);
         } else if (is_kquant(fmt)) {
             const Plan p = plan_kquant(rows, cols, chunk, MODE == kSwiglu, row_bytes);
@@ -816,7 +957,7 @@ int rta_dequant(int fmt, const void* src, int64_t n, float* out, rta_stream_t st
 
 size_t rta_gemv_workspace_bytes(int fmt, int rows, int cols, int batch) {
     if (rows <= 0 || cols <= 0 || batch <= 0 || ((is_kquant(fmt) || is_tiled(fmt)) && cols % 256)) return 0;
-    return projection_ws(fmt, rows, cols, batch < kMaxBatchTile ? batch : kMaxBatchTile, false);
+    return projection_ws(fmt, rows, cols, batch, false);
 }
 
 int rta_gemv(int fmt, const void* w, int rows, int cols, const float* x, int batch, float* y, int epilogue,
@@ -829,7 +970,8 @@ int rta_gemv(int fmt, const void* w, int rows, int cols, const float* x, int bat
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(y) % 4 ||
         reinterpret_cast<uintptr_t>(workspace) % 256)
         return RTA_ERR_ALIGN;
-    if (workspace_bytes < rta_gemv_workspace_bytes(fmt, rows, cols, batch)) return RTA_ERR_WORKSPACE;
+    // (a workspace sized for a smaller batch still serves the narrow tiles)
+    if (workspace_bytes < rta_gemv_workspace_bytes(fmt, rows, cols, one_tile(batch))) return RTA_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     if (epilogue == RTA_EPI_STORE)
         return run_projection<kStore>(fmt, w, nullptr, rows, cols, x, batch, y, nullptr, nullptr, nullptr, workspace,
@@ -838,14 +980,19 @@ int rta_gemv(int fmt, const void* w, int rows, int cols, const float* x, int bat
                                        workspace_bytes, s);
 }
 
-size_t rta_gemv_remap_workspace_bytes(int fmt, const rta_remap* remap, int rows, int cols, int batch) {
+// Bytes of a remapped readout of `batch` rows whose projection workspace covers inner_batch.
+static size_t remap_ws(int fmt, const rta_remap* remap, int rows, int cols, int batch, int inner_batch) {
     Remap m;
     int need = 0;
     if (batch <= 0 || check_remap(remap, INT_MAX, rows, cols, &m, &need)) return 0;
-    const size_t inner = rta_gemv_workspace_bytes(fmt, need, cols, batch);
+    const size_t inner = rta_gemv_workspace_bytes(fmt, need, cols, inner_batch);
     if (m.mode == RTA_REMAP_NONE) return inner;
     if ((is_kquant(fmt) || is_tiled(fmt)) && cols % 256) return 0;
     return (m.moves_rows() ? floats256((int64_t)batch * need) : floats256((int64_t)batch * cols)) + inner;
+}
+
+size_t rta_gemv_remap_workspace_bytes(int fmt, const rta_remap* remap, int rows, int cols, int batch) {
+    return remap_ws(fmt, remap, rows, cols, batch, batch);
 }
 
 int rta_gemv_remap(int fmt, const void* w, int src_rows, int rows, int cols, const rta_remap* remap, const float* x,
@@ -864,7 +1011,7 @@ int rta_gemv_remap(int fmt, const void* w, int src_rows, int rows, int cols, con
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(y) % 4 ||
         reinterpret_cast<uintptr_t>(workspace) % 256)
         return RTA_ERR_ALIGN;
-    if (workspace_bytes < rta_gemv_remap_workspace_bytes(fmt, remap, rows, cols, batch)) return RTA_ERR_WORKSPACE;
+    if (workspace_bytes < remap_ws(fmt, remap, rows, cols, batch, one_tile(batch))) return RTA_ERR_WORKSPACE;
     if (!workspace) return RTA_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -896,9 +1043,8 @@ size_t rta_mlp_workspace_bytes(int fmt_g, int fmt_d, int hidden, int inter, int 
     if (hidden <= 0 || inter <= 0 || batch <= 0) return 0;
     if (((is_kquant(fmt_g) || is_tiled(fmt_g)) && hidden % 256) || ((is_kquant(fmt_d) || is_tiled(fmt_d)) && inter % 256))
         return 0;
-    const int tile = batch < kMaxBatchTile ? batch : kMaxBatchTile;
-    const size_t a = projection_ws(fmt_g, inter, hidden, tile, true);
-    const size_t b = projection_ws(fmt_d, hidden, inter, tile, false);
+    const size_t a = projection_ws(fmt_g, inter, hidden, batch, true);
+    const size_t b = projection_ws(fmt_d, hidden, inter, batch, false);
     return a > b ? a : b;
 }
 
@@ -916,7 +1062,8 @@ int rta_mlp_swiglu(int fmt_g, const void* wg, int fmt_u, const void* wu, int fmt
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(act) % 16 ||
         reinterpret_cast<uintptr_t>(y) % 4 || reinterpret_cast<uintptr_t>(workspace) % 256)
         return RTA_ERR_ALIGN;
-    if (workspace_bytes < rta_mlp_workspace_bytes(fmt_g, fmt_d, hidden, inter, batch)) return RTA_ERR_WORKSPACE;
+    if (workspace_bytes < rta_mlp_workspace_bytes(fmt_g, fmt_d, hidden, inter, one_tile(batch)))
+        return RTA_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     rc = run_projection<kSwiglu>(fmt_g, wg, wu, inter, hidden, x, batch, act, nullptr, nullptr, nullptr, workspace,
                                  workspace_bytes, s);
@@ -938,7 +1085,7 @@ int rta_swiglu(int fmt, const void* wg, const void* wu, int hidden, int inter, c
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(act) % 16 ||
         reinterpret_cast<uintptr_t>(workspace) % 256)
         return RTA_ERR_ALIGN;
-    if (workspace_bytes < rta_mlp_workspace_bytes(fmt, fmt, hidden, inter, batch)) return RTA_ERR_WORKSPACE;
+    if (workspace_bytes < rta_mlp_workspace_bytes(fmt, fmt, hidden, inter, one_tile(batch))) return RTA_ERR_WORKSPACE;
     return run_projection<kSwiglu>(fmt, wg, wu, inter, hidden, x, batch, act, nullptr, nullptr, nullptr, workspace,
                                    workspace_bytes, (hipStream_t)stream);
 }
@@ -948,7 +1095,7 @@ size_t rta_lm_head_workspace_bytes(int fmt, int vocab, int hidden, int batch) {
     if ((is_kquant(fmt) || is_tiled(fmt)) && hidden % 256) return 0;
     // per-task maxima [batch][vocab] (upper bound), then the matrix-core scratch of one tile
     const size_t maxima = ((size_t)vocab * (size_t)batch * sizeof(float) + 255) & ~(size_t)255;
-    return maxima + projection_ws(fmt, vocab, hidden, batch < kMaxBatchTile ? batch : kMaxBatchTile, false);
+    return maxima + projection_ws(fmt, vocab, hidden, batch, false);
 }
 
 int rta_lm_head(int fmt, const void* w, int vocab, int hidden, const float* h, int batch, float margin, float* logits,
@@ -970,8 +1117,9 @@ int lm_head_rownorm(int fmt, const void* w, int vocab, int hidden, const float* 
     if (batch <= 0) return RTA_ERR_SHAPE;
     if (!(margin >= 0.0f) || !(margin < 1.0f)) return RTA_ERR_RANGE;
     const size_t maxima = ((size_t)vocab * (size_t)batch * sizeof(float) + 255) & ~(size_t)255;
-    const size_t mma = projection_ws(fmt, vocab, hidden, batch < kMaxBatchTile ? batch : kMaxBatchTile, false);
-    if (!workspace || workspace_bytes < rta_lm_head_workspace_bytes(fmt, vocab, hidden, batch)) return RTA_ERR_WORKSPACE;
+    if (!workspace || workspace_bytes < maxima + projection_ws(fmt, vocab, hidden, one_tile(batch), false))
+        return RTA_ERR_WORKSPACE;
+    const size_t mma = workspace_bytes - maxima;
     if (reinterpret_cast<uintptr_t>(h) % 16 || reinterpret_cast<uintptr_t>(logits) % 4 ||
         reinterpret_cast<uintptr_t>(ids) % 4 || reinterpret_cast<uintptr_t>(workspace) % 256)
         return RTA_ERR_ALIGN;
@@ -981,7 +1129,8 @@ int lm_head_rownorm(int fmt, const void* w, int vocab, int hidden, const float* 
     int b0 = 0;
     while (b0 < batch) {
         const bool cores = is_kquant(fmt) && mma_batch((int64_t)vocab * hidden, batch);
-        const int cap = (cores || is_tiled(fmt)) ? kMaxBatchTile : 8;
+        const bool wide = !rn.part && use_wide(fmt, vocab, hidden, batch, false, scratch, mma);
+        const int cap = wide ? kWideBatch : (cores || is_tiled(fmt)) ? kMaxBatchTile : 8;
         const int chunk = batch - b0 < cap ? batch - b0 : cap;
         int ntasks = 0, rpt = 1;
         RowNorm rc_rn = rn;

@@ -157,11 +157,11 @@ struct Work {
 // count up to the whole in-projection's, and a readout's workspace does not grow steadily
 // with its rows (fewer row tiles get more K slabs).  Within one run of row counts that
 // share a plan (the same number of 16- or 32-row tiles) the slab partials grow with the
-// rows, so the multiples of 16 bound every count.  Cached per (hidden, batch tile, rows).
+// rows, so the multiples of 16 bound every count.  Cached per (hidden, batch, rows).
 size_t parts_ws_bytes(int D, int B, int rows_max) {
     static std::mutex mu;
     static std::map<std::tuple<int, int, int>, size_t> memo;
-    const auto key = std::make_tuple(D, std::min(B, 32), rows_max);
+    const auto key = std::make_tuple(D, B, rows_max);
     {
         std::lock_guard<std::mutex> g(mu);
         const auto it = memo.find(key);

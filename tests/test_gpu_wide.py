@@ -1,0 +1,105 @@
+"""The readouts of more than one matrix-core batch tile (over 32 rows) at the edges of the
+wide kernel's blocks: 64 / 128-row batch blocks, partial row tiles and row blocks, one and
+several K slabs, batches past one launch (256 rows), GGUF rows (also Q6_K rows that start 2
+bytes into a dword) and packed tiles, every epilogue; and that a workspace sized for a batch
+of 32 is still accepted and gives the same results to rounding.
+
+Bar: max|gpu - ref| <= 1e-5 + 1e-3 max|ref| per tensor against the fp64 oracle; between the
+two paths 1e-5 of the peak (both sum the same exact products in fp32)."""
+import numpy as np
+import pytest
+
+import oracle as orc
+from conftest import assert_close
+from rta import _lib, ops, synth
+from rta._lib import TILED
+
+pytestmark = pytest.mark.gpu
+REL, ABS = 1e-3, 1e-5
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+
+
+def matrix(rng, fmt, rows, cols, packed, shift=0):
+    import torch
+    w = synth.random_matrix(rng, fmt, rows, cols)
+    if packed:
+        return w, ops.pack(fmt, dev(w), rows, cols), fmt | TILED
+    held = torch.zeros(w.size + shift, dtype=torch.uint8, device="cuda:0")
+    held[shift:] = dev(w.reshape(-1))
+    return w, held[shift:], fmt
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("fmt", [orc.Q4_K, orc.Q6_K])
+@pytest.mark.parametrize("rows,cols,batch", [(16, 256, 33), (17, 512, 64), (300, 768, 65), (1000, 2304, 128),
+                                             (4096, 1024, 129), (777, 256, 256), (130, 512, 300), (8200, 2048, 200)])
+def test_wide_readout(fmt, packed, rows, cols, batch):
+    rng = np.random.default_rng(rows + 3 * cols + 5 * batch + fmt)
+    w, wd, f = matrix(rng, fmt, rows, cols, packed, shift=2 if fmt == orc.Q6_K and not packed else 0)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[1] *= 1e3
+    x[2] *= 1e-3
+    x[batch - 1] = 0
+    ref = orc.gemv_f64(fmt, w, rows, cols, x)
+    y = ops.gemv(f, wd, rows, cols, dev(x))
+    for b in range(batch):
+        assert_close(y[b].cpu().numpy(), ref[b], f"row {b}")
+    y0 = rng.standard_normal((batch, rows)).astype(np.float32)
+    ya = ops.gemv(f, wd, rows, cols, dev(x), y=dev(y0), accumulate=True)
+    assert_close(ya.cpu().numpy(), ref + y0, "accumulated")
+    # a workspace sized for 32 rows keeps the narrow tiles
+    need = ops.gemv_workspace_bytes(f, rows, cols, 32)
+    small = np.zeros(max(need, 1), np.uint8)
+    assert ops.gemv_workspace_bytes(f, rows, cols, batch) >= need
+    yn = ops.gemv(f, wd, rows, cols, dev(x), workspace=dev(small))
+    peak = float(np.abs(ref).max())
+    assert float((yn - y).abs().max()) <= 1e-5 * peak
+    if need:
+        with pytest.raises(_lib.RtaError):
+            ops.gemv(f, wd, rows, cols, dev(x), workspace=dev(small[:need - 1]))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("hidden,inter,batch", [(512, 1536, 100), (2048, 6144, 256), (768, 1024, 257)])
+def test_wide_mlp(packed, hidden, inter, batch):
+    rng = np.random.default_rng(hidden + inter + batch)
+    (g, gd, f), (u, ud, _) = (matrix(rng, orc.Q4_K, inter, hidden, packed) for _ in range(2))
+    d, dd, fd = matrix(rng, orc.Q6_K, hidden, inter, packed)
+    x = rng.standard_normal((batch, hidden)).astype(np.float32)
+    act, y = ops.mlp_swiglu((f, f, fd), gd, ud, dd, hidden, inter, dev(x))
+    ract, ry = orc.mlp_swiglu((orc.Q4_K, orc.Q4_K, orc.Q6_K), g, u, d, hidden, inter, x)
+    assert_close(act.cpu().numpy(), ract, "activation")
+    assert_close(y.cpu().numpy(), ry, "output")
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("vocab,hidden,batch", [(3001, 512, 33), (20011, 1024, 65), (9000, 256, 260)])
+def test_wide_lm_head(packed, vocab, hidden, batch):
+    rng = np.random.default_rng(vocab + hidden + batch)
+    w, wd, f = matrix(rng, orc.Q6_K, vocab, hidden, packed)
+    h = (rng.standard_normal((batch, hidden)) * 2).astype(np.float32)
+    logits, ids = ops.lm_head(f, wd, vocab, hidden, dev(h))
+    lg, ids = logits.cpu().numpy(), ids.cpu().numpy().view(np.uint32)
+    ref = orc.gemv_f64(orc.Q6_K, w, vocab, hidden, h)
+    assert_close(lg, ref, "logits")
+    for b in range(batch):
+        assert int(ids[b]) == orc.argmax_margin_f32(lg[b], 1e-4), b
+
+
+@pytest.mark.parametrize("fmt", [orc.Q4_K, orc.Q6_K])
+@pytest.mark.parametrize("rows,cols", [(700, 4096), (2064, 768)])
+def test_rows_of_wide_calls_do_not_depend_on_the_batch(fmt, rows, cols):
+    """Bitwise: packed calls of 33 to 64 rows against calls of 17 to 32; within the classes
+    (64, 128] and above 128 rows, across launches of 256, on packed tiles and GGUF rows."""
+    rng = np.random.default_rng(rows + cols + fmt)
+    x = dev(rng.standard_normal((600, cols)).astype(np.float32))
+    for packed in (False, True):
+        _, wd, f = matrix(rng, fmt, rows, cols, packed)
+        y = {n: ops.gemv(f, wd, rows, cols, x[:n]).cpu().numpy() for n in (20, 32, 33, 64, 65, 128, 129, 257, 600)}
+        for a, b in ((20, 64), (32, 33), (65, 128), (129, 600), (257, 600)):
+            if packed or a > 64:
+                assert np.array_equal(y[a], y[b][:a]), (packed, a, b)
