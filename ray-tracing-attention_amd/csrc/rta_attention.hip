@@ -356,9 +356,11 @@ __device__ __forceinline__ void attn_plan_wave(const AttnArgs& a) {
         int before, total;
         scan(t, before, total);
         if (s < a.nseq) a.plan[s] = (int32_t)(carry + before);
-        // The run of workgroups whose first tile lies in each sequence, written by the whole
-        // wave sequence by sequence (one lane writing its own sequence's run took 16 us for one
-        // sequence of 512 workgroups, and takes 4.7 so, launch included)
+        // The run of workgroups whose first tile lies in each sequence: short runs by the
+        // sequence's own lane, runs much longer than the sequences are many by the whole wave,
+        // sequence by sequence.  One lane alone took 16.2 us for a sequence of 512 workgroups,
+        // the wave 4.7 (launch included); 27 sequences of 2 workgroups the other way round,
+        // 2 us more for the call
         const int64_t first = carry + before, end = first + t;
         int w0 = 0, w1 = 0;   // at most nwg workgroups
         if (t > 0) {
@@ -366,9 +368,14 @@ __device__ __forceinline__ void attn_plan_wave(const AttnArgs& a) {
             w1 = (int)((end * P + T - 1) / T);
         }
         const int here = a.nseq - s0 < kWave ? a.nseq - s0 : kWave;
-        for (int i = 0; i < here; ++i) {   // uniform
-            const int wb = __builtin_amdgcn_readlane(w1, i);
-            for (int w = __builtin_amdgcn_readlane(w0, i) + lane; w < wb; w += kWave) a.plan[a.nseq + 1 + w] = s0 + i;
+        if (__builtin_amdgcn_ballot_w64(w1 - w0 > 4 * here) == 0) {
+            for (int w = w0; w < w1; ++w) a.plan[a.nseq + 1 + w] = s;
+        } else {
+            for (int i = 0; i < here; ++i) {   // uniform
+                const int wb = __builtin_amdgcn_readlane(w1, i);
+                for (int w = __builtin_amdgcn_readlane(w0, i) + lane; w < wb; w += kWave)
+                    a.plan[a.nseq + 1 + w] = s0 + i;
+            }
         }
         carry += total;
     }
