@@ -370,7 +370,7 @@ def readout_name(fmt_name, rows, cols, batch, packed, pair=False):
         return f"gemv_b1_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
     weights = rows * cols * (2 if pair else 1)
     if batch >= 5 or (batch >= 3 and weights >= 1 << 25) or (batch >= 2 and weights >= 1 << 27):
-        return f"xprep_kernel + gemm_mfma_kernel<{fmt_name}> (GGUF rows, matrix cores)"
+        return f"gemm_tiled_kernel<{fmt_name}> (GGUF rows, matrix cores)"
     return f"gemv_kquant_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
 
 

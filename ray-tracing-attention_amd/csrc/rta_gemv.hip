@@ -300,55 +300,16 @@ __host__ __device__ constexpr bool mma_batch(int64_t weights, int batch) {
     return (batch >= 5 && weights >= kMmaAnyWeights) || (batch >= 3 && weights >= kMmaMidWeights) ||
            (batch >= 2 && weights >= kMmaTallWeights);
 }
-constexpr int kMfmaRT = 2;         // 16-row tiles per wave
-
 struct MmaPlan {
     int nbt, total_rows, ntg, nslab, sb_per_slab, wgs_per_slab, grid;
-    size_t x_bytes, part_bytes;
+    size_t part_bytes;
 };
 
-// Work split of one projection over a batch tile: K slabs that fit the LDS, doubled
-// while the (tile, slab) units would leave waves idle.  Independent of the device so
-// that workspace sizes are host queries.
-static MmaPlan plan_mfma(int rows, int cols, int nbt, bool dual) {
-    MmaPlan p{};
-    p.nbt = nbt;
-    p.total_rows = dual ? 2 * rows : rows;
-    p.ntg = (p.total_rows + 16 * kMfmaRT - 1) / (16 * kMfmaRT);
-    const int nsbt = cols / 256;
-    const int sbmax = kSlabRowSb / (16 * nbt);
-    int nslab = (nsbt + sbmax - 1) / sbmax;
-    while (nslab < nsbt && (int64_t)p.ntg * nslab < (int64_t)kPlanCUs * kGemmWaves) nslab *= 2;
-    if (nslab > nsbt) nslab = nsbt;
-    p.sb_per_slab = (nsbt + nslab - 1) / nslab;
-    p.nslab = (nsbt + p.sb_per_slab - 1) / p.sb_per_slab;
-    int wps = (kPlanCUs + p.nslab - 1) / p.nslab;
-    const int need = (p.ntg + kGemmWaves - 1) / kGemmWaves;
-    p.wgs_per_slab = wps < need ? wps : need;
-    p.grid = p.nslab * p.wgs_per_slab;
-    p.x_bytes = (size_t)kMaxBatchTile * cols * 2 * 2                 // hi, lo
-              + (size_t)kMaxBatchTile * nsbt * 64                    // group-sum operands
-              + (size_t)kMaxBatchTile * nsbt * sizeof(float);        // 1 / scale
-    p.x_bytes = (p.x_bytes + 255) & ~(size_t)255;
-    p.part_bytes = p.nslab > 1 ? (size_t)p.nslab * kMaxBatchTile * p.total_rows * sizeof(float) : 0;
-    return p;
-}
-
-static GemmX carve_x(void* ws, int cols) {
-    uint8_t* b = static_cast<uint8_t*>(ws);
-    GemmX x;
-    const size_t n = (size_t)kMaxBatchTile * cols;
-    const size_t nsbt = cols / 256;
-    x.hi = reinterpret_cast<_Float16*>(b);
-    x.lo = reinterpret_cast<_Float16*>(b + 2 * n);
-    x.g = reinterpret_cast<h8_t*>(b + 4 * n);
-    x.inv = reinterpret_cast<float*>(b + 4 * n + (size_t)kMaxBatchTile * nsbt * 64);
-    return x;
-}
-
-// Work split of a projection over packed tiles: 16-row tiles are shared out to the
-// waves of each K slab in balanced contiguous ranges and multiplied in pairs (the
-// gate and up tiles of one row range in kSwiglu).
+// Work split of a projection over 16-row tiles (packed, or of GGUF rows): they are shared
+// out to the waves of each K slab in balanced contiguous ranges and multiplied in pairs (the
+// gate and up tiles of one row range in kSwiglu).  K slabs fit the LDS, doubled while the
+// (tile pair, slab) units would leave waves idle.  Independent of the device so that
+// workspace sizes are host queries.
 static MmaPlan plan_tiled(int rows, int cols, int nbt, bool dual) {
     MmaPlan p{};
     p.nbt = nbt;
@@ -368,7 +329,6 @@ static MmaPlan plan_tiled(int rows, int cols, int nbt, bool dual) {
     const int need = (units + kGemmWaves - 1) / kGemmWaves;
     p.wgs_per_slab = wps < need ? wps : need;
     p.grid = p.nslab * p.wgs_per_slab;
-    p.x_bytes = 0;   // x is prepared in LDS by the kernel
     p.part_bytes = p.nslab > 1 ? (size_t)p.nslab * kMaxBatchTile * p.total_rows * sizeof(float) : 0;
     return p;
 }
@@ -376,13 +336,9 @@ static MmaPlan plan_tiled(int rows, int cols, int nbt, bool dual) {
 // Bytes of workspace one projection needs for its batch tiles of at most 32 rows (0 when
 // the VALU paths serve it); covers batch tiles of either width.
 static size_t narrow_ws(int fmt, int rows, int cols, int batch, bool dual) {
-    if (is_tiled(fmt)) {
-        const MmaPlan a = plan_tiled(rows, cols, 1, dual), b = plan_tiled(rows, cols, 2, dual);
-        return a.x_bytes + (a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes);
-    }
-    if (!(fmt == RTA_Q4_K || fmt == RTA_Q6_K) || !mma_batch((int64_t)rows * cols * (dual ? 2 : 1), batch)) return 0;
-    const MmaPlan a = plan_mfma(rows, cols, 1, dual), b = plan_mfma(rows, cols, 2, dual);
-    return a.x_bytes + (a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes);
+    if (!is_tiled(fmt) && !(is_kquant(fmt) && mma_batch((int64_t)rows * cols * (dual ? 2 : 1), batch))) return 0;
+    const MmaPlan a = plan_tiled(rows, cols, 1, dual), b = plan_tiled(rows, cols, 2, dual);
+    return a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes;
 }
 
 // Work split of wide_kernel (rta_wide.hpp) for a call of `batch` rows in launches of up to
@@ -433,10 +389,9 @@ static size_t wide_x_bytes(int cols, int n) {
     return (b + 255) & ~(size_t)255;
 }
 
-// Workspace of the wide launches of a call of `batch` rows (0: it makes none).  GGUF rows up
-// to 64 stay on the narrow tiles, whose order of summation over K is another.
+// Workspace of the wide launches of a call of `batch` rows (0: it makes none).
 static size_t wide_ws(int fmt, int rows, int cols, int batch, bool dual) {
-    if (!wide_format(fmt) || batch <= (is_tiled(fmt) ? kMaxBatchTile : 64)) return 0;
+    if (!wide_format(fmt) || batch <= kMaxBatchTile) return 0;
     const WidePlan p = plan_wide(rows, cols, batch, dual);
     const int n = batch < kWideBatch ? batch : kWideBatch;
     return wide_x_bytes(cols, n) +
@@ -462,53 +417,18 @@ static void launch_reduce(dim3 grid, const float* part, int nslab, int rows, int
 }
 
 template <int FMT, int NBT, int MODE>
-static void launch_gemm(const MmaPlan& p, const Launch& l, const GemmX& xp, float* part, float* pmax,
-                        hipStream_t s) {
-    hipLaunchKernelGGL((xprep_kernel<FMT == RTA_Q6_K ? kXpQ6Row : kXpQ4Row>), dim3(l.cols / 256, 8 * NBT), dim3(64), 0, s, l.x, l.cols,
-                       l.batch, xp);
-    hipLaunchKernelGGL((gemm_mfma_kernel<FMT, kMfmaRT, NBT, MODE>), dim3(p.grid), dim3(64 * kGemmWaves), 0, s, l.w,
-                       l.w2, l.row_bytes, l.rows, l.cols, xp, l.batch, l.y, part, pmax, p.sb_per_slab,
-                       p.wgs_per_slab);
-}
-
-// One batch tile (<= 32 rows): xprep -> MFMA GEMM (-> fixed-order slab reduce).
-// For kLogits, pmax receives per-task maxima [batch][*ntasks_out], tasks of
-// *rpt_out rows.
-template <int MODE>
-static hipError_t run_mfma(int fmt, const Launch& l, void* ws, float* pmax, int* ntasks_out, int* rpt_out,
-                           hipStream_t s) {
-    const int nbt = l.batch > 16 ? 2 : 1;
-    const MmaPlan p = plan_mfma(l.rows, l.cols, nbt, MODE == kSwiglu);
-    GemmX xp = carve_x(ws, l.cols);
-    float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + p.x_bytes);
-    if (fmt == RTA_Q4_K) {
-        if (nbt == 1) launch_gemm<RTA_Q4_K, 1, MODE>(p, l, xp, part, pmax, s);
-        else launch_gemm<RTA_Q4_K, 2, MODE>(p, l, xp, part, pmax, s);
-    } else {
-        if (nbt == 1) launch_gemm<RTA_Q6_K, 1, MODE>(p, l, xp, part, pmax, s);
-        else launch_gemm<RTA_Q6_K, 2, MODE>(p, l, xp, part, pmax, s);
-    }
-    if (p.nslab > 1) {
-        const dim3 rg((l.rows + 255) / 256, l.batch);
-        launch_reduce<MODE>(rg, part, p.nslab, l.rows, l.batch, l.y, pmax, s);
-        if (ntasks_out) *ntasks_out = (int)rg.x;
-        if (rpt_out) *rpt_out = 256;
-    } else {
-        if (ntasks_out) *ntasks_out = p.ntg;
-        if (rpt_out) *rpt_out = 16 * kMfmaRT;
-    }
-    return hipGetLastError();
-}
-
-template <int FMT, int NBT, int MODE>
 static void launch_tiled(const MmaPlan& p, const Launch& l, float* part, float* pmax, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_tiled_kernel<FMT, NBT, MODE>), dim3(p.wgs_per_slab, p.nslab), dim3(64 * kGemmWaves), 0,
-                       s, l.w, l.w2, l.rows, l.cols, l.x, l.batch, l.y, part, pmax, p.sb_per_slab, p.wgs_per_slab,
-                       l.rn);
+    const dim3 g(p.wgs_per_slab, p.nslab), b(64 * kGemmWaves);
+    if (l.row_bytes)   // GGUF rows
+        hipLaunchKernelGGL((gemm_tiled_kernel<FMT, NBT, MODE, true>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows,
+                           l.cols, l.x, l.batch, l.y, part, pmax, p.sb_per_slab, p.wgs_per_slab, l.rn);
+    else
+        hipLaunchKernelGGL((gemm_tiled_kernel<FMT, NBT, MODE, false>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows,
+                           l.cols, l.x, l.batch, l.y, part, pmax, p.sb_per_slab, p.wgs_per_slab, l.rn);
 }
 
-// One batch tile (<= 32 rows) over packed weights: the tiled GEMM prepares x in LDS
-// itself; with several K slabs, gemm_reduce_kernel adds the partials in slab order.
+// One batch tile (<= 32 rows) over packed tiles or GGUF rows: the tiled GEMM prepares x in
+// LDS itself; with several K slabs, gemm_reduce_kernel adds the partials in slab order.
 template <int MODE>
 static hipError_t run_tiled(int fmt, const Launch& l, void* ws, float* pmax, int* ntasks_out, int* rpt_out,
                             hipStream_t s) {
@@ -644,12 +564,10 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
         if (wide) {
             e = run_wide<MODE>(fmt, plan_wide(rows, cols, whole, MODE == kSwiglu), l, ws, l.partial, ntasks_out,
                                rows_per_task_out, s);
-        } else if (tiled) {
-            if (!ws || ws_bytes < narrow_ws(fmt, rows, cols, chunk, MODE == kSwiglu)) return RTA_ERR_WORKSPACE;
+        } else if (tiled || mma) {
+            const size_t need = narrow_ws(fmt, rows, cols, one_tile(whole), MODE == kSwiglu);
+            if ((!ws && (need || tiled)) || ws_bytes < need) return RTA_ERR_WORKSPACE;
             e = run_tiled<MODE>(fmt, l, ws, l.partial, ntasks_out, rows_per_task_out, s);
-        } else if (mma) {
-            if (!ws || ws_bytes < narrow_ws(fmt, rows, cols, chunk, MODE == kSwiglu)) return RTA_ERR_WORKSPACE;
-            e = run_mfma<MODE>(fmt, l, ws, l.partial, ntasks_out, rows_per_task_out, s);
         } else if (is_kquant(fmt)) {
             const Plan p = plan_kquant(rows, cols, chunk, MODE == kSwiglu, row_bytes);
             if (ntasks_out) *ntasks_out = p.ntasks;
@@ -694,7 +612,6 @@ static MmaPlan plan_packed(int rows, int cols, int nbt, bool dual) {
     const int need = (units + kPkWaves - 1) / kPkWaves;
     p.wgs_per_slab = wps < need ? wps : need;
     p.grid = p.nslab * p.wgs_per_slab;
-    p.x_bytes = 0;
     p.part_bytes = p.nslab > 1 ? (size_t)p.nslab * kMaxBatchTile * p.total_rows * sizeof(float) : 0;
     return p;
 }

@@ -34,7 +34,9 @@
 //         8 (s/2) + 2 (m/2) + s%2
 // and x is read from LDS at exactly those columns (k-permuted inside each 8 as in
 // the row-layout path).  The minimum (Q4_K) / -32 offset (Q6_K) terms use group
-// sums of x that xprep_kernel lays out per lane segment to match.
+// sums of x laid out per lane segment to match (XStage):
+//   Q4_K  segment s = [hi, lo of 32-group 2s, hi, lo of 2s+1, 0, 0, 0, 0]
+//   Q6_K  segment s = [hi, lo of 16-group g(q)] for q = 0..3, g(q) = 8 (s/2) + 2 q + s%2
 #pragma once
 #include "rta_gemm.hpp"
 #include "rta_remap.hpp"
@@ -239,8 +241,94 @@ __device__ __forceinline__ uint32_t h2dup_scaled(uint32_t v, float c) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, x));
 }
 
+// Where a lane finds its share of a 16-row tile's superblock, in packed tiles or in GGUF
+// rows: offsets from the tile's bytes (tiled) or from the lane's own row's block.  Either way
+// the lane gets the same values (TileFmt::Raw).  Q6_K GGUF blocks are 2-byte aligned: their
+// 16-byte runs are read as the five dwords around them, from the aligned address at or below
+// (every dword overlaps the block), and funnelled; unaligned 16-byte loads took 19.9 us where
+// the dwords take 13.5 (2048x6144 readout of 8 rows).
+template <int FMT>
+struct LaneSource;
+
+__device__ __forceinline__ uint4 load16(const uint8_t* p) {
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
+template <>
+struct LaneSource<RTA_Q4_K> {
+    using Raw = TileFmt<RTA_Q4_K>::Raw;
+    int oh, oq, dq, stride;   // header and quant offsets, second quant run, superblock stride
+    __device__ __forceinline__ LaneSource(bool tiled, int lane) {
+        const int li = lane & 15, s = lane >> 4;
+        oh = tiled ? 16 * li : 0;
+        oq = tiled ? 256 + 16 * lane : 16 + 32 * s;
+        dq = tiled ? 1024 : 16;
+        stride = tiled ? TileFmt<RTA_Q4_K>::kBytes : 144;
+    }
+    __device__ __forceinline__ void load(const uint8_t* p, Raw& r) const {
+        r.hdr = load16(p + oh);
+        r.q0 = load16(p + oq);
+        r.q1 = load16(p + oq + dq);
+    }
+};
+
+template <>
+struct LaneSource<RTA_Q6_K> {
+    using Raw = TileFmt<RTA_Q6_K>::Raw;
+    bool tiled;
+    int os, od, oa, db, oh, stride;
+    __device__ __forceinline__ LaneSource(bool tiled_, int lane) : tiled(tiled_) {
+        const int li = lane & 15, s = lane >> 4, h = s >> 1, o = 16 * (s & 1);
+        os = tiled ? 16 * li : 192;
+        od = tiled ? 256 + 2 * li : 208;
+        oa = tiled ? 288 + 16 * lane : 64 * h + o;
+        db = tiled ? 1024 : 32;
+        oh = tiled ? 2336 + 16 * lane : 128 + 32 * h + o;
+        stride = tiled ? TileFmt<RTA_Q6_K>::kBytes : 210;
+    }
+    // 16 bytes at p, mis (0 or 2) bytes past a dword boundary
+    __device__ static __forceinline__ uint4 run(const uint8_t* p, uint32_t mis) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(p - mis);
+        uint4 v;
+        __builtin_memcpy(&v, w, 16);
+        const uint32_t x = w[4];
+        return uint4{funnel(v.x, v.y, mis), funnel(v.y, v.z, mis), funnel(v.z, v.w, mis), funnel(v.w, x, mis)};
+    }
+    __device__ __forceinline__ void load(const uint8_t* p, Raw& r) const {
+        r.d = *reinterpret_cast<const uint16_t*>(p + od);
+        if (tiled) {
+            r.sc = load16(p + os);
+            r.a = load16(p + oa);
+            r.b = load16(p + oa + db);
+            r.h = load16(p + oh);
+        } else {   // every run starts a multiple of 16 bytes into the block
+            const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 3u);
+            r.sc = run(p + os, mis);
+            r.a = run(p + oa, mis);
+            r.b = run(p + oa + db, mis);
+            r.h = run(p + oh, mis);
+        }
+    }
+};
+
+// Scales and minima of groups 2 s and 2 s + 1 from a GGUF Q4_K header (bytes 4..15 in
+// h.y, h.z, h.w; resident_quant.glsl:10-19): groups 0-3 in the low six bits of bytes j and
+// j + 4, groups 4-7 in nibbles of byte j + 4 with their high bits above the former.
+__device__ __forceinline__ void q4k_row_scale_min(const uint4& h, int s, uint32_t& sc0, uint32_t& sc1, uint32_t& m0,
+                                                  uint32_t& m1) {
+    const uint32_t sh = 16u * (uint32_t)(s & 1);
+    const uint32_t y = h.y >> sh, z = h.z >> sh, w = h.w >> sh;
+    const bool low = s < 2;
+    sc0 = low ? y & 63u : (w & 15u) | ((y >> 2) & 48u);
+    sc1 = low ? (y >> 8) & 63u : ((w >> 8) & 15u) | ((y >> 10) & 48u);
+    m0 = low ? z & 63u : ((w >> 4) & 15u) | ((z >> 2) & 48u);
+    m1 = low ? (z >> 8) & 63u : ((w >> 12) & 15u) | ((z >> 10) & 48u);
+}
+
 // Prepares x rows [0, 16 NBT) over superblocks [sb0, sb0 + nsb) straight into LDS,
-// in the tiled-readout layouts (kXpQ4Tile / kXpQ6Tile of xprep_kernel): per (row,
+// in the layouts above: per (row,
 // superblock) a power-of-two scale s with max|x s| in [2^13, 2^14), x s as binary16
 // hi + lo (k-permuted inside each 8-value segment), the group sums of x s (/32 for
 // Q4_K, /16 for Q6_K) as hi + lo, and 1/s (0 for rows >= batch).  32 threads per
@@ -338,9 +426,13 @@ struct XStage {
 // Units of work: pairs of 16-row tiles (t = 0, 1).  In kSwiglu the pair is (gate
 // tile T, up tile T) of one unit T; otherwise tiles (a + 2u, a + 2u + 1) of the
 // wave's contiguous tile range [a, b), the second one absent at an odd end.
-template <int FMT, int NBT, int MODE>
+// ROWS: w and w2 are GGUF rows of row_bytes bytes instead of packed tiles (tile t: rows 16 t
+// to 16 t + 15, the last row repeated past the end), otherwise the same kernel, so both
+// layouts sum in the same order.
+template <int FMT, int NBT, int MODE, bool ROWS>
 __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
-    const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, const int rows, const int cols,
+    const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, const int64_t row_bytes, const int rows,
+    const int cols,
     const float* __restrict__ x, const int batch, float* __restrict__ y, float* __restrict__ part,
     float* __restrict__ pmax, const int sb_per_slab, const int wgs_per_slab, const RowNorm rn) {
     constexpr bool kQ4 = FMT == RTA_Q4_K;
@@ -366,6 +458,7 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
 
     const int s = lane >> 4, li = lane & 15;
     const Q4kSegment seg(s);
+    const LaneSource<FMT> rows_at(false, lane);   // ROWS
     const int total_rows = MODE == kSwiglu ? 2 * rows : rows;
     const int ntile = (rows + 15) >> 4;
 
@@ -388,8 +481,13 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
         int t0, t1;
         tiles_of(lu, t0, t1);
         const int64_t sb = sb0 + lsb;
-        F::load(w + ((int64_t)t0 * nsbt + sb) * F::kBytes, lane, dst[0]);
-        F::load((MODE == kSwiglu ? w2 : w) + ((int64_t)t1 * nsbt + sb) * F::kBytes, lane, dst[1]);
+        if constexpr (ROWS) {
+            rows_at.load(w + min(16 * t0 + li, rows - 1) * row_bytes + sb * F::kBlock, dst[0]);
+            rows_at.load((MODE == kSwiglu ? w2 : w) + min(16 * t1 + li, rows - 1) * row_bytes + sb * F::kBlock, dst[1]);
+        } else {
+            F::load(w + ((int64_t)t0 * nsbt + sb) * F::kBytes, lane, dst[0]);
+            F::load((MODE == kSwiglu ? w2 : w) + ((int64_t)t1 * nsbt + sb) * F::kBytes, lane, dst[1]);
+        }
         if (lit < nit - 1) {
             ++lit;
             if (++lsb == nsb) {
@@ -456,7 +554,8 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
                 dC[t] = half_lo(h.x) * 16384.0f;     // codes carry 2^-14
                 dM[t] = half_hi(h.x) * 32.0f;        // group sums are staged / 32
                 uint32_t sc0, m0, sc1, m1;
-                q4k_tile_scale_min(h, seg, sc0, sc1, m0, m1);
+                if constexpr (ROWS) q4k_row_scale_min(h, s, sc0, sc1, m0, m1);
+                else q4k_tile_scale_min(h, seg, sc0, sc1, m0, m1);
                 slo[t] = h2dup_scaled(sc0, 1024.0f);
                 shi[t] = h2dup_scaled(sc1, 64.0f);
                 bm[t] = __builtin_bit_cast(h8_t, uint4{h2dup_scaled(m0, 1.0f), h2dup_scaled(m1, 1.0f), 0u, 0u});

@@ -17,7 +17,7 @@
 // Arithmetic per superblock, operand values and scales are those of the narrow readouts
 // (rta_gemm.hpp): x s as hi + lo binary16, exact code x sub-block scale products, the group
 // sums in one more MFMA, then d, the minimum / offset and 1 / s on the fp32 results.
-// GGUF rows and packed tiles differ only in where a lane's bytes lie (WideSource).
+// GGUF rows and packed tiles differ only in where a lane's bytes lie (LaneSource).
 //
 // Bound: matrix cores (two MFMAs per weight tile, 16 rows and 32 columns) where the grid
 // fills the chip; per superblock of TN = 8, NB = 2 a wave issues 272 MFMAs (4352 cycles)
@@ -120,72 +120,6 @@ __global__ void __launch_bounds__(512) wide_xprep_kernel(const float* __restrict
     if (tid < 64) p.g[at * 64 + tid] = __builtin_bit_cast(uint4, gs[tid & 15][tid >> 4]);
 }
 
-// A lane's bytes of row tile T: a base pointer (its row's first superblock, or the tile's)
-// and lane offsets.  Loads are 16 bytes; Q6_K GGUF blocks are 2-byte aligned and read as
-// they lie (unaligned global loads of exactly the bytes needed).
-template <int FMT>
-struct WideSource;
-
-__device__ __forceinline__ uint4 load16(const uint8_t* p) {
-    uint4 v;
-    __builtin_memcpy(&v, p, 16);
-    return v;
-}
-
-template <>
-struct WideSource<RTA_Q4_K> {
-    struct Raw { uint4 hdr, q0, q1; };
-    int oh, oq, dq, stride;   // header and quant offsets, second quant run, superblock stride
-    __device__ __forceinline__ WideSource(bool tiled, int lane) {
-        const int li = lane & 15, s = lane >> 4;
-        oh = tiled ? 16 * li : 0;
-        oq = tiled ? 256 + 16 * lane : 16 + 32 * s;
-        dq = tiled ? 1024 : 16;
-        stride = tiled ? TileFmt<RTA_Q4_K>::kBytes : 144;
-    }
-    __device__ __forceinline__ void load(const uint8_t* p, Raw& r) const {
-        r.hdr = load16(p + oh);
-        r.q0 = load16(p + oq);
-        r.q1 = load16(p + oq + dq);
-    }
-};
-
-template <>
-struct WideSource<RTA_Q6_K> {
-    struct Raw { uint4 sc, a, b, h; uint32_t d; };
-    int os, od, oa, db, oh, stride;
-    __device__ __forceinline__ WideSource(bool tiled, int lane) {
-        const int li = lane & 15, s = lane >> 4, h = s >> 1, o = 16 * (s & 1);
-        os = tiled ? 16 * li : 192;
-        od = tiled ? 256 + 2 * li : 208;
-        oa = tiled ? 288 + 16 * lane : 64 * h + o;
-        db = tiled ? 1024 : 32;
-        oh = tiled ? 2336 + 16 * lane : 128 + 32 * h + o;
-        stride = tiled ? TileFmt<RTA_Q6_K>::kBytes : 210;
-    }
-    __device__ __forceinline__ void load(const uint8_t* p, Raw& r) const {
-        r.sc = load16(p + os);
-        r.d = *reinterpret_cast<const uint16_t*>(p + od);
-        r.a = load16(p + oa);
-        r.b = load16(p + oa + db);
-        r.h = load16(p + oh);
-    }
-};
-
-// Scales and minima of groups 2 s and 2 s + 1 from a GGUF Q4_K header (bytes 4..15 in
-// h.y, h.z, h.w; resident_quant.glsl:10-19): groups 0-3 in the low six bits of bytes j and
-// j + 4, groups 4-7 in nibbles of byte j + 4 with their high bits above the former.
-__device__ __forceinline__ void q4k_row_scale_min(const uint4& h, int s, uint32_t& sc0, uint32_t& sc1, uint32_t& m0,
-                                                  uint32_t& m1) {
-    const uint32_t sh = 16u * (uint32_t)(s & 1);
-    const uint32_t y = h.y >> sh, z = h.z >> sh, w = h.w >> sh;
-    const bool low = s < 2;
-    sc0 = low ? y & 63u : (w & 15u) | ((y >> 2) & 48u);
-    sc1 = low ? (y >> 8) & 63u : ((w >> 8) & 15u) | ((y >> 10) & 48u);
-    m0 = low ? z & 63u : ((w >> 4) & 15u) | ((z >> 2) & 48u);
-    m1 = low ? (z >> 8) & 63u : ((w >> 12) & 15u) | ((z >> 10) & 48u);
-}
-
 struct WideArgs {
     const uint8_t* w;
     const uint8_t* w2;       // DUAL: the up matrix
@@ -214,7 +148,7 @@ struct WideMeta {
 template <int FMT, bool DUAL, int NB, int TN>
 __global__ void __launch_bounds__(kWideThreads, 2) wide_kernel(const WideArgs a) {
     constexpr bool kQ4 = FMT == RTA_Q4_K, kSplit = kWideSplit<NB>;
-    using Source = WideSource<FMT>;
+    using Source = LaneSource<FMT>;
     using Raw = typename Source::Raw;
     constexpr int DT = (2 * TN + 7) / 8;   // tiles a wave decodes (the last only while they last)
     __shared__ WideLds<TN> buf0;

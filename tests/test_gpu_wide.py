@@ -93,7 +93,7 @@ def test_wide_lm_head(packed, vocab, hidden, batch):
 @pytest.mark.parametrize("fmt", [orc.Q4_K, orc.Q6_K])
 @pytest.mark.parametrize("rows,cols", [(700, 4096), (2064, 768)])
 def test_rows_of_wide_calls_do_not_depend_on_the_batch(fmt, rows, cols):
-    """Bitwise: packed calls of 33 to 64 rows against calls of 17 to 32; within the classes
+    """Bitwise: calls of 33 to 64 rows against calls of 17 to 32; within the classes
     (64, 128] and above 128 rows, across launches of 256, on packed tiles and GGUF rows."""
     rng = np.random.default_rng(rows + cols + fmt)
     x = dev(rng.standard_normal((600, cols)).astype(np.float32))
@@ -101,5 +101,4 @@ def test_rows_of_wide_calls_do_not_depend_on_the_batch(fmt, rows, cols):
         _, wd, f = matrix(rng, fmt, rows, cols, packed)
         y = {n: ops.gemv(f, wd, rows, cols, x[:n]).cpu().numpy() for n in (20, 32, 33, 64, 65, 128, 129, 257, 600)}
         for a, b in ((20, 64), (32, 33), (65, 128), (129, 600), (257, 600)):
-            if packed or a > 64:
-                assert np.array_equal(y[a], y[b][:a]), (packed, a, b)
+            assert np.array_equal(y[a], y[b][:a]), (packed, a, b)
