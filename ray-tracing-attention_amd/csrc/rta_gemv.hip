@@ -586,9 +586,8 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
 }
 
 // ---- readouts of a staged x image (rta_packed.hpp), used by the decode step -------
-// Kernel shape: tiles per wave and superblock, waves per workgroup, superblocks of
-// weights in flight per wave.
-constexpr int kPkTpw = 2, kPkWaves = 8, kPkDepth = 2;
+// Kernel shape: tiles per wave and superblock, waves per workgroup.
+constexpr int kPkTpw = 2, kPkWaves = 8;
 
 // Work split: units of kPkTpw tiles (kSwiglu: gate and up tiles of the same rows) are
 // shared out to the waves of each K slab in balanced contiguous ranges.  The K range is
@@ -686,7 +685,7 @@ int swiglu_image(int fmt, const float* part, int nslab, int width, int batch, vo
 template <int FMT, int NBT, int MODE>
 static void launch_packed(const MmaPlan& p, const uint8_t* w, const uint8_t* w2, int rows, int cols, const void* img,
                           int batch, float* y, float* part, const RowNorm& rn, hipStream_t s) {
-    hipLaunchKernelGGL((gemm_packed_kernel<FMT, NBT, MODE, kPkTpw, kPkWaves, kPkDepth>),
+    hipLaunchKernelGGL((gemm_packed_kernel<FMT, NBT, MODE, kPkTpw, kPkWaves>),
                        dim3(p.wgs_per_slab, p.nslab), dim3(64 * kPkWaves), 0, s, w, w2, rows, cols, static_cast<const XImage<NBT>*>(img), batch, y,
                        part, p.sb_per_slab, p.wgs_per_slab, rn);
 }

@@ -16,8 +16,8 @@
 // gemm_packed_kernel: one workgroup per compute unit and K slab; each wave takes a
 // balanced contiguous range of units of TPW tiles (kSwiglu: TPW/2 gate tiles and the
 // TPW/2 up tiles of the same rows) and, per superblock, reads the x operands of a
-// column offset from LDS once for all TPW tiles.  The weights of the next DEPTH - 1
-// superblocks are in flight in registers while one is multiplied.  The slab's images
+// column offset from LDS once for all TPW tiles.  The weights of the next superblock are in
+// flight in registers while one is multiplied.  The slab's images
 // reach LDS by direct global -> LDS loads (global_load_lds_dwordx4).  Tile format and
 // operand layouts are those of rta_tiled.hpp.
 #pragma once
@@ -211,7 +211,7 @@ __global__ void __launch_bounds__(256) swiglu_image_kernel(const float* __restri
     image_row<FMT, NBT>(img[sb], b, live, v, lane);
 }
 
-template <int FMT, int NBT, int MODE, int TPW, int NWAVES, int DEPTH>
+template <int FMT, int NBT, int MODE, int TPW, int NWAVES>
 __global__ void __launch_bounds__(64 * NWAVES) gemm_packed_kernel(
     const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2, const int rows, const int cols,
     const XImage<NBT>* __restrict__ xi, const int batch, float* __restrict__ y, float* __restrict__ part,
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(64 * NWAVES) gemm_packed_kernel(
     // The slab's x images go to LDS first, by direct global -> LDS loads (lane l of a
     // wave's instruction lands at the wave's LDS base + 16 l, so a wave moves 64
     // consecutive 16-byte words per instruction without a register round trip); all of
-    // them are in flight at once, with DEPTH - 1 superblocks of weights issued behind
+    // them are in flight at once, with one superblock of weights issued behind
     // them.  They are issued before the work split is worked out: a kernel starts with
     // cold instruction and scalar caches, and the loads are the long pole.
     constexpr int kThreads = 64 * NWAVES;
@@ -303,11 +303,8 @@ __global__ void __launch_bounds__(64 * NWAVES) gemm_packed_kernel(
             }
         }
     };
-    Raw buf[DEPTH][TPW];
-    if (nit > 0) {
-#pragma unroll
-        for (int d = 0; d < DEPTH - 1; ++d) load_next(buf[d]);
-    }
+    Raw cur[TPW], nxt[TPW];
+    if (nit > 0) load_next(cur);
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the direct loads have landed
     __syncthreads();
 
@@ -505,70 +502,80 @@ __global__ void __launch_bounds__(64 * NWAVES) gemm_packed_kernel(
     const int head = cu;                      // the wave's first unit ...
     const bool head_shared = csb != 0;        // ... began in an earlier wave
     f4_t hacc[TPW][NBT];                      // its partial sums, for that wave
-    for (int it0 = 0; it0 < nit; it0 += DEPTH) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            const int it = it0 + d;
-            load_next(buf[(d + DEPTH - 1) % DEPTH]);
-            if (it < nit) {
-                take_turns(wave, it);
-                compute(csb, buf[d]);
-                if (csb == nsb - 1) {
-                    if (head_shared && cu == head) {
-#pragma unroll
-                        for (int t = 0; t < TPW; ++t)
-#pragma unroll
-                            for (int bt = 0; bt < NBT; ++bt) {
-                                hacc[t][bt] = acc[t][bt];
-                                acc[t][bt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                            }
-                    } else {
-                        finish(cu);
-                    }
-                }
-                if (++csb == nsb) {
-                    csb = 0;
-                    ++cu;
-                }
-            }
-        }
-    }
-    // units left open: the head piece of a unit that ends inside this wave's range holds
-    // only a middle part (it is the head partial), or the wave owns an unfinished unit
-    const bool open = nit > 0 && csb != 0;
-    const bool mid = open && head_shared && cu == head;
-    if (mid) {
-#pragma unroll
-        for (int t = 0; t < TPW; ++t)
-#pragma unroll
-            for (int bt = 0; bt < NBT; ++bt) hacc[t][bt] = acc[t][bt];
-    }
-    // hand the head partials over through LDS (the x images are no longer read)
+    // The items, then one pass (it == nit) that hands the head partials over and closes the
+    // wave's last unit.  One copy each of the multiplication and of finish(), the buffers
+    // rotated by register moves: a kernel's code is fetched cold at every launch, and a body
+    // unrolled over the two buffers with finish() three times was 24.6 KB against 13.2 (gate/up
+    // pair in the batch-32 step 22.1 -> 21.9 us; with gemm_tiled_kernel's likewise, the step
+    // 3838 -> 3776 us and a 2048-wide MLP of 8 rows 25.9 -> 23.2).
     constexpr int kSlot = TPW * NBT * 4 * 64;   // floats per wave
     static_assert(NWAVES * kSlot * sizeof(float) <= sizeof(sx), "partial slots fit in the x images");
     float* slots = reinterpret_cast<float*>(sx);
-    __syncthreads();
-    if (head_shared && nit > 0) {
+#pragma clang loop unroll(disable)
+    for (int it = 0; it <= nit; ++it) {
+        bool done = false;
+        if (it < nit) {
+            load_next(nxt);
+            take_turns(wave, it);
+            compute(csb, cur);
+            if (csb == nsb - 1) {
+                if (head_shared && cu == head) {
 #pragma unroll
-        for (int t = 0; t < TPW; ++t)
+                    for (int t = 0; t < TPW; ++t)
 #pragma unroll
-            for (int bt = 0; bt < NBT; ++bt)
+                        for (int bt = 0; bt < NBT; ++bt) {
+                            hacc[t][bt] = acc[t][bt];
+                            acc[t][bt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                        }
+                } else {
+                    done = true;
+                }
+            }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) slots[wave * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane] = hacc[t][bt][e];
-    }
-    __syncthreads();
-    if (open && !mid) {   // the owner adds the pieces of the later waves in wave order
-        const int end = (cu - wa + 1) * nsb;   // items of the unit end here
-        for (int wv = wave + 1; wv < NWAVES && item0(wv) < end; ++wv) {
-            if (item0(wv + 1) == item0(wv)) continue;   // (a wave without items holds no piece)
+            for (int t = 0; t < TPW; ++t) cur[t] = nxt[t];
+        } else {
+            // units left open: the head piece of a unit that ends inside this wave's range holds
+            // only a middle part (it is the head partial), or the wave owns an unfinished unit
+            const bool open = nit > 0 && csb != 0;
+            const bool mid = open && head_shared && cu == head;
+            if (mid) {
 #pragma unroll
-            for (int t = 0; t < TPW; ++t)
+                for (int t = 0; t < TPW; ++t)
 #pragma unroll
-                for (int bt = 0; bt < NBT; ++bt)
+                    for (int bt = 0; bt < NBT; ++bt) hacc[t][bt] = acc[t][bt];
+            }
+            // hand the head partials over through LDS (the x images are no longer read)
+            __syncthreads();
+            if (head_shared && nit > 0) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[t][bt][e] += slots[wv * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane];
+                for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                    for (int bt = 0; bt < NBT; ++bt)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            slots[wave * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane] = hacc[t][bt][e];
+            }
+            __syncthreads();
+            if (open && !mid) {   // the owner adds the pieces of the later waves in wave order
+                const int end = (cu - wa + 1) * nsb;   // items of the unit end here
+                for (int wv = wave + 1; wv < NWAVES && item0(wv) < end; ++wv) {
+                    if (item0(wv + 1) == item0(wv)) continue;   // (a wave without items holds no piece)
+#pragma unroll
+                    for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                        for (int bt = 0; bt < NBT; ++bt)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                acc[t][bt][e] += slots[wv * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane];
+                }
+                done = true;
+            }
         }
-        finish(cu);
+        if (done) finish(cu);
+        if (++csb == nsb) {
+            csb = 0;
+            ++cu;
+        }
     }
 }
 

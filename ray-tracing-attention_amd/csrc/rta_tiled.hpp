@@ -497,12 +497,8 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
         }
     };
 
-    constexpr int DEPTH = 2;   // one superblock loads while the current one multiplies
-    Raw buf[DEPTH][2];
-    if (nit > 0) {
-#pragma unroll
-        for (int d = 0; d < DEPTH - 1; ++d) load_next(buf[d]);
-    }
+    Raw cur[2], nxt[2];   // one superblock loads while the current one multiplies
+    if (nit > 0) load_next(cur);
     xs.store(sm, batch, nsb, rn);
     __syncthreads();
 
@@ -708,22 +704,21 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
             for (int bt = 0; bt < NBT; ++bt) acc[t][bt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
     };
 
+    // one copy of the body, the buffers rotated by register moves: the code is fetched cold at
+    // every launch
     int cu = 0, csb = 0;   // (unit, superblock) being multiplied
-    for (int it0 = 0; it0 < nit; it0 += DEPTH) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            const int it = it0 + d;
-            load_next(buf[(d + DEPTH - 1) % DEPTH]);
-            if (it < nit) {
-                take_turns(wave, it);
-                compute(csb, buf[d]);
-                if (csb == nsb - 1) finish(cu);
-                if (++csb == nsb) {
-                    csb = 0;
-                    ++cu;
-                }
-            }
+#pragma clang loop unroll(disable)
+    for (int it = 0; it < nit; ++it) {
+        load_next(nxt);
+        take_turns(wave, it);
+        compute(csb, cur);
+        if (csb == nsb - 1) finish(cu);
+        if (++csb == nsb) {
+            csb = 0;
+            ++cu;
         }
+        cur[0] = nxt[0];
+        cur[1] = nxt[1];
     }
 }
 
