@@ -410,7 +410,7 @@ __global__ void __launch_bounds__(64 * NW) recurrent_mix_kernel(
     __shared__ float z_s[hd];
     __shared__ float gates_s[2];
     __shared__ float o_s[hd];
-    __shared__ float red[NW];
+    __shared__ float norm_s[2][2], out_s[2];
     const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int W = heads * hd, W3 = 3 * W, KW = key_heads * hd, hk = h % key_heads;
@@ -504,18 +504,21 @@ __global__ void __launch_bounds__(64 * NW) recurrent_mix_kernel(
             gates_s[1] = detector_sigmoid(gb);
         }
     }
-    // L2 norm of q and k over the head (waves 0 and 1 hold its 128 coordinates)
+    // L2 norm of q and k over the head (waves 0 and 1 hold its 128 coordinates), both behind
+    // one barrier
+    if (wave < 2) {
 #pragma unroll
-    for (int part = 0; part < 2; ++part) {
-        const float ss = wave_sum(y[part] * y[part]);
-        __syncthreads();
-        if (lane == 0 && wave < 2) red[wave] = ss;
-        __syncthreads();
-        y[part] *= 1.0f / sqrtf(red[0] + red[1] + eps);
+        for (int part = 0; part < 2; ++part) {
+            const float ss = wave_sum(y[part] * y[part]);
+            if (lane == 0) norm_s[part][wave] = ss;
+        }
     }
+    __syncthreads();
     if (tid < hd) {
 #pragma unroll
-        for (int part = 0; part < 3; ++part) qkv_s[part][tid] = y[part];
+        for (int part = 0; part < 2; ++part)
+            qkv_s[part][tid] = y[part] * (1.0f / sqrtf(norm_s[part][0] + norm_s[part][1] + eps));
+        qkv_s[2][tid] = y[2];
     }
     __syncthreads();
 
@@ -548,11 +551,17 @@ __global__ void __launch_bounds__(64 * NW) recurrent_mix_kernel(
         for (int j = 0; j < kWords; ++j) o_s[rbase + j * rstep] = o[j] * scale;
     }
     __syncthreads();
-    // op 15: gated RMSNorm of o
+    // op 15: gated RMSNorm of o (waves 0 and 1)
     const float v = tid < hd ? o_s[tid] : 0.0f;
-    const float ss = block_sum<NW>(v * v, red);
-    const float inv = 1.0f / sqrtf(ss / (float)hd + eps);
-    if (tid < hd) out[(int64_t)b * out_stride + h * hd + tid] = v * inv * norm_w[h * hd + tid] * silu(z_s[tid]);
+    if (wave < 2) {
+        const float ss = wave_sum(v * v);
+        if (lane == 0) out_s[wave] = ss;
+    }
+    __syncthreads();
+    if (tid < hd) {
+        const float inv = 1.0f / sqrtf((out_s[0] + out_s[1]) / (float)hd + eps);
+        out[(int64_t)b * out_stride + h * hd + tid] = v * inv * norm_w[h * hd + tid] * silu(z_s[tid]);
+    }
 }
 
 int recurrent_mix(const float* proj, int64_t slab_stride, int row_stride, int nslab, int key_heads, const float* ext_a,
