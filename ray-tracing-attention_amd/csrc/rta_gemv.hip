@@ -203,7 +203,7 @@ struct Launch {
     float* partial;
     int batch;
     RowNorm rn;   // packed readouts only
-    XNorm xn;     // batch-1 readouts only
+    XNorm xn;     // batch-1 and wide readouts only
 };
 
 template <int FMT, int R, int MODE, int KW>
@@ -362,7 +362,9 @@ static WidePlan plan_wide(int rows, int cols, int batch, bool dual) {
     const double total = 16.0 * ntile * (dual ? 2 : 1);
     double least = 0.0;
     for (int tn = 4; tn <= 8; tn += 2) {
-        if (nb == 1 && tn == 6) continue;   // not built: the narrow batch block is bound by its start
+        // up to 64 rows the call is bound by its start, not its tiles: the smallest blocks, two
+        // to a compute unit (8-tile waves: the 64-sequence step 1073 us against 986)
+        if (nb == 1 && tn != 4) continue;
         const int per = dual ? tn : 2 * tn, nblk = (ntile + per - 1) / per;
         for (int ns = 1; ns <= nsbt; ++ns) {
             const int spb = (nsbt + ns - 1) / ns;
@@ -458,8 +460,7 @@ template <int FMT, bool DUAL>
 static void launch_wide(const WidePlan& p, const WideArgs& a, hipStream_t s) {
     const dim3 g(p.nblk, (a.batch + 64 * p.nb - 1) / (64 * p.nb), p.nslab), b(kWideThreads);
     if (p.nb == 1) {
-        if (p.tn == 4) hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 1, 4>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 1, 8>), g, b, 0, s, a);
+        hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 1, 4>), g, b, 0, s, a);
     } else {
         if (p.tn == 4) hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 2, 4>), g, b, 0, s, a);
         else if (p.tn == 6) hipLaunchKernelGGL((wide_kernel<FMT, DUAL, 2, 6>), g, b, 0, s, a);
@@ -468,10 +469,12 @@ static void launch_wide(const WidePlan& p, const WideArgs& a, hipStream_t s) {
 }
 
 template <int FMT>
-static void launch_wide_xprep(const WidePlan& p, const float* x, int cols, int batch, const WideX& to, hipStream_t s) {
-    const dim3 g(cols / 256, (batch + 15) / 16), b(512);
-    if (kWideSplit<2> && p.nb == 2) hipLaunchKernelGGL((wide_xprep_kernel<FMT, true>), g, b, 0, s, x, cols, batch, to);
-    else hipLaunchKernelGGL((wide_xprep_kernel<FMT, false>), g, b, 0, s, x, cols, batch, to);
+static void launch_wide_xprep(const WidePlan& p, const Launch& l, const WideX& to, hipStream_t s) {
+    const dim3 g(l.cols / 256, (l.batch + 15) / 16), b(512);
+    if (kWideSplit<2> && p.nb == 2)
+        hipLaunchKernelGGL((wide_xprep_kernel<FMT, true>), g, b, 0, s, l.x, l.cols, l.batch, to, l.xn.w, l.xn.eps);
+    else
+        hipLaunchKernelGGL((wide_xprep_kernel<FMT, false>), g, b, 0, s, l.x, l.cols, l.batch, to, l.xn.w, l.xn.eps);
 }
 
 // Up to kWideBatch rows of a call with plan p: x fragments -> wide_kernel (-> fixed-order
@@ -499,10 +502,10 @@ static hipError_t run_wide(int fmt, const WidePlan& p, const Launch& l, void* ws
     a.sb_per_slab = p.sb_per_slab;
     a.mode = MODE;
     if ((fmt & 0xff) == RTA_Q4_K) {
-        launch_wide_xprep<RTA_Q4_K>(p, l.x, l.cols, l.batch, a.x, s);
+        launch_wide_xprep<RTA_Q4_K>(p, l, a.x, s);
         launch_wide<RTA_Q4_K, kDual>(p, a, s);
     } else {
-        launch_wide_xprep<RTA_Q6_K>(p, l.x, l.cols, l.batch, a.x, s);
+        launch_wide_xprep<RTA_Q6_K>(p, l, a.x, s);
         launch_wide<RTA_Q6_K, kDual>(p, a, s);
     }
     if (p.nslab > 1) {
@@ -534,7 +537,6 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
                           size_t ws_bytes, hipStream_t s, int path_batch = 0, const RowNorm& rn = RowNorm{},
                           const XNorm& xn = XNorm{}) {
     if (rn.part && !is_tiled(fmt)) return RTA_ERR_FORMAT;   // only the packed readout applies it
-    if (xn.w && !b1_norm_fusable(fmt, cols, batch)) return RTA_ERR_FORMAT;   // only the batch-1 readout
     const bool tiled = is_tiled(fmt);
     const int64_t row_bytes = tiled ? 0 : host::row_bytes(fmt, cols);
     int b0 = 0;
@@ -544,6 +546,8 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
                      mma_batch((int64_t)rows * cols * (MODE == kSwiglu ? 2 : 1), path_batch > 0 ? path_batch : batch);
     const int whole = path_batch > 0 ? path_batch : batch;
     const bool wide = !rn.part && use_wide(fmt, rows, cols, whole, MODE == kSwiglu, ws, ws_bytes);
+    // only the batch-1 and wide readouts take the norm themselves
+    if (xn.w && !wide && !b1_norm_fusable(fmt, cols, whole)) return RTA_ERR_FORMAT;
     while (b0 < batch) {
         const int cap = wide ? kWideBatch : (mma || tiled) ? kMaxBatchTile : 8;
         const int chunk = batch - b0 < cap ? batch - b0 : cap;
@@ -782,6 +786,13 @@ int projection_store(int fmt, const void* w, int rows, int cols, const float* x,
     if (rc) return rc;
     return run_projection<kStore>(fmt, w, nullptr, rows, cols, x, batch, y, nullptr, nullptr, nullptr, ws, ws_bytes, s,
                                   0, rn, xn);
+}
+
+// The wide readout's x preparation takes the norm where re-reading the rows once per
+// superblock costs less than a launch of its own (64 rows: 4.7 us).
+bool wide_norm_fusable(int fmt, int rows, int cols, int batch, bool dual, size_t ws_bytes) {
+    const size_t need = wide_ws(fmt, rows, cols, batch, dual);
+    return need && ws_bytes >= need && cols <= 4096;
 }
 
 bool b1_norm_fusable(int fmt, int cols, int batch) {

@@ -26,6 +26,9 @@ struct XNorm {
     float eps = 0.0f;
 };
 bool b1_norm_fusable(int fmt, int cols, int batch);
+// Likewise over the rows of a batch of more than 32 (the wide readout; ws_bytes: the
+// workspace the call will pass).
+bool wide_norm_fusable(int fmt, int rows, int cols, int batch, bool dual, size_t ws_bytes);
 
 // y = W x (rta_gemv with the STORE epilogue) with a deferred RMSNorm factor (rn) or the
 // batch-1 readout's own RMSNorm (xn).

@@ -381,12 +381,15 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
     // GGUF-row K-quant readout takes the norm itself (xn; its x is then w.hidden).
     RowNorm rn{};
     XNorm xn{};
-    auto norm = [&](const float* nw, int f, bool keep_fp32) -> int {
+    // Above 32 rows the wide readout takes it too (rows, dual: the consumer's matrix).
+    auto norm = [&](const float* nw, int f, bool keep_fp32, int rows, bool dual) -> int {
         rn = RowNorm{};
         xn = XNorm{};
         const float* part = static_cast<const float*>(w.gemm_ws);
         int rc;
-        if (!keep_fp32 && !pending && b1_norm_fusable(f, d.D, B)) {
+        if (!keep_fp32 && !pending &&
+            (b1_norm_fusable(f, d.D, B) ||
+             (nw && host::aligned(nw, 16) && wide_norm_fusable(f, rows, d.D, B, dual, w.gemm_bytes)))) {
             xn = XNorm{nw, eps};
             return capture_residual();
         }
@@ -420,7 +423,7 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
             fusable = fusable && b1_norm_fusable(lw.in_fmt[i], d.D, B);
         }
         if (sum != rows) return RTA_ERR_SHAPE;
-        RTA_TRY(norm(lw.norm_in, fusable ? lw.in_fmt[0] : RTA_F32, keep_fp32));
+        RTA_TRY(norm(lw.norm_in, fusable ? lw.in_fmt[0] : RTA_F32, keep_fp32, rows, false));
         int off = 0;
         for (int i = 0; i < lw.in_parts; ++i) {
             const int n = lw.in_rows[i], f = lw.in_fmt[i];
@@ -452,7 +455,7 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
             if (lw.in_parts > 0) {
                 RTA_TRY(in_parts(lw, d.rows_full, false));
             } else {
-                RTA_TRY(norm(lw.norm_in, fi, false));
+                RTA_TRY(norm(lw.norm_in, fi, false, d.rows_full, false));
                 if (imaged(fi))
                     RTA_TRY(image_readout(fi, kReadStore, lw.w_in, nullptr, d.rows_full, d.D, w.ximg, B, w.proj,
                                           false, w.gemm_ws, w.gemm_bytes, s, &ns, rn));
@@ -489,7 +492,7 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
             if (lw.in_parts > 0) {
                 RTA_TRY(in_parts(lw, rows, ext));
             } else {
-                RTA_TRY(norm(lw.norm_in, fi, ext));
+                RTA_TRY(norm(lw.norm_in, fi, ext, rows, false));
                 if (imaged(fi))
                     RTA_TRY(image_readout(fi, kReadStore, lw.w_in, nullptr, rows, d.D, w.ximg, B, w.proj, false,
                                           w.gemm_ws, w.gemm_bytes, s, &ns, rn));
@@ -531,7 +534,7 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
             ++lr;
         }
         // op 1 index 1, then the SwiGLU MLP with the residual add (executeMLP)
-        RTA_TRY(norm(lw.norm_post, fgu, false));
+        RTA_TRY(norm(lw.norm_post, fgu, false, d.FF, true));
         bool down_done = false;
         if (imaged(fgu)) {
             // a packed down projection reads the SwiGLU of the gate/up K slabs as its x
@@ -563,7 +566,10 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
         rn = RowNorm{};
         xn = XNorm{};
         const float* part = static_cast<const float*>(w.gemm_ws);
-        if (!pending && b1_norm_fusable(fl, d.D, B)) {
+        const size_t maxima = ((size_t)d.V * B * sizeof(float) + 255) & ~(size_t)255;   // (lm_ws: then the readout's)
+        if (!pending && (b1_norm_fusable(fl, d.D, B) ||
+                         (host::aligned(weights->norm_final, 16) &&
+                          wide_norm_fusable(fl, d.V, d.D, B, false, w.lm_bytes - maxima)))) {
             xn = XNorm{weights->norm_final, eps};
         } else if (fused(fl) && d.D <= 4096) {
             RTA_TRY(residual_norm_deferred(w.hidden, part, pending, weights->norm_final, B, d.D, w.normed, w.rms, s));

@@ -52,8 +52,13 @@ __device__ __forceinline__ int wide_step(bool q4, bool split, int m) {
 }
 
 // Block: 16 rows x 32 threads of 8 columns, one superblock (grid: superblocks x row tiles).
+// With nw, x is a residual row and its RMSNorm (op 1: x nw / sqrt(mean(x^2) + eps)) is taken
+// here, every block summing its rows' squares itself: the rows are read once per superblock
+// from the cache, for the launch of a norm kernel saved (64-sequence step of 17 norms: 986 ->
+// 964 us).
 template <int FMT, bool SPLIT>
-__global__ void __launch_bounds__(512) wide_xprep_kernel(const float* __restrict__ x, int cols, int batch, WideX p) {
+__global__ void __launch_bounds__(512) wide_xprep_kernel(const float* __restrict__ x, int cols, int batch, WideX p,
+                                                         const float* __restrict__ nw, float eps) {
     constexpr bool kQ4 = FMT == RTA_Q4_K;
     __shared__ uint4 frag[16][64];
     __shared__ h8_t gs[16][4];
@@ -67,6 +72,25 @@ __global__ void __launch_bounds__(512) wide_xprep_kernel(const float* __restrict
         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = c.x; v[5] = c.y; v[6] = c.z; v[7] = c.w;
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = live ? v[i] : 0.0f;
+    }
+    if (nw) {   // uniform
+        const float4* xr = reinterpret_cast<const float4*>(x + (int64_t)min(row, batch - 1) * cols);
+        float ss = 0.0f;
+#pragma unroll 8
+        for (int i = t; i < cols >> 2; i += 32) {
+            const float4 a = xr[i];
+            ss += (a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w);
+        }
+        ss += dpp_mov<0xB1>(ss);
+        ss += dpp_mov<0x4E>(ss);
+        ss += dpp_mov<0x141>(ss);
+        ss += dpp_mov<0x140>(ss);
+        const float inv = 1.0f / sqrtf(add_xor16(ss) / (float)cols + eps);
+        const float4* g = reinterpret_cast<const float4*>(nw + sb * 256 + 8 * t);
+        const float4 g0 = g[0], g1 = g[1];
+        const float gw[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = v[i] * inv * gw[i];
     }
     float m = 0.0f;
 #pragma unroll
