@@ -361,17 +361,15 @@ def w_mlp(torch, args, orc):
 
 def readout_name(fmt_name, rows, cols, batch, packed, pair=False):
     """The kernel a projection readout runs (the library's dispatch, for the bench line's
-    label): packed tiles on the matrix cores; GGUF rows on the batch-1 readout, the
-    vector-ALU batch readout, or the matrix cores from batch 5 (3 at 2^25+ weights, 2 at
+    label): packed tiles on the matrix cores; GGUF rows on the vector-ALU
+    readout, or the matrix cores from batch 5 (3 at 2^25+ weights, 2 at
     2^27+ weights, a SwiGLU pair counting both matrices)."""
     if packed:
         return f"gemm_tiled_kernel<{fmt_name}> (packed tiles, matrix cores)"
-    if batch == 1:
-        return f"gemv_b1_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
     weights = rows * cols * (2 if pair else 1)
     if batch >= 5 or (batch >= 3 and weights >= 1 << 25) or (batch >= 2 and weights >= 1 << 27):
         return f"gemm_tiled_kernel<{fmt_name}> (GGUF rows, matrix cores)"
-    return f"gemv_kquant_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
+    return f"gemv_b1_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
 
 
 def w_lm_head(torch, args, orc):

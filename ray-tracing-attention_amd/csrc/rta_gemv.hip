@@ -150,18 +150,18 @@ static bool is_kquant(int fmt) { return fmt == RTA_Q4_K || fmt == RTA_Q6_K; }
 constexpr int kPlanCUs = 256;      // CUs the work split is planned for (MI355X)
 
 struct Plan {
-    bool b1;          // batch-1 kernel
+    bool b1;          // batch-1 kernel (a grid row per batch row)
     int nb, r, kw, lpr, ntasks, grid, block, rows_per_task;
 };
 
-// Launch plan of one K-quant projection over `batch` (<= 8) x rows; row_bytes of one
+// Launch plan of one K-quant projection over `batch` (<= 4) x rows; row_bytes of one
 // matrix row (both matrices' rows are streamed in the dual case).
 static Plan plan_kquant(int rows, int cols, int batch, bool dual, int64_t row_bytes) {
     Plan p{};
     const int S = cols / 64;
-    p.b1 = batch == 1 && S <= 4 * kWave;
+    p.b1 = batch <= 4 && S <= 4 * kWave;
     if (p.b1) {
-        p.nb = 1;
+        p.nb = batch;
         p.r = dual ? 1 : 2;
         p.kw = S <= kWave ? 1 : (S + kWave - 1) / kWave;
         p.lpr = S >= kWave ? kWave : pow2ceil(S);
@@ -180,9 +180,8 @@ static Plan plan_kquant(int rows, int cols, int batch, bool dual, int64_t row_by
         p.grid = blocks < cap ? blocks : (int)cap;
         return p;
     }
-    p.nb = batch <= 1 ? 1 : batch <= 2 ? 2 : batch <= 4 ? 4 : 8;
-    p.r = p.nb >= 8 ? 2 : 4;
-    if (dual) p.r = p.r / 2 > 0 ? p.r / 2 : 1;
+    p.nb = batch <= 1 ? 1 : batch <= 2 ? 2 : 4;
+    p.r = dual ? 2 : 4;
     p.kw = 1;
     p.lpr = S >= kWave ? kWave : pow2ceil(S);
     p.rows_per_task = (kWave / p.lpr) * p.r;
@@ -215,7 +214,7 @@ static void launch_b1(const Plan& p, const Launch& l, hipStream_t s) {
             hipFuncAttributeMaxDynamicSharedMemorySize, b1_lds_bytes(4 * kWave));
         (void)attr;   // a failure surfaces as the launch error
     }
-    hipLaunchKernelGGL((gemv_b1_kernel<FMT, R, MODE, KW>), dim3(p.grid), dim3(p.block), lds, s, l.w, l.w2,
+    hipLaunchKernelGGL((gemv_b1_kernel<FMT, R, MODE, KW>), dim3(p.grid, p.nb), dim3(p.block), lds, s, l.w, l.w2,
                        l.row_bytes, l.rows, l.cols, l.x, l.y, l.partial, p.lpr, p.ntasks, l.xn.w, l.xn.eps);
 }
 
@@ -241,8 +240,7 @@ static void launch_kquant_fmt(const Plan& p, const Launch& l, hipStream_t s) {
     switch (p.nb) {
     case 1: hipLaunchKernelGGL((gemv_kquant_kernel<FMT, 1, dual ? 2 : 4, MODE>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows, l.cols, l.x, l.y, l.partial, l.batch, p.lpr, p.ntasks); break;
     case 2: hipLaunchKernelGGL((gemv_kquant_kernel<FMT, 2, dual ? 2 : 4, MODE>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows, l.cols, l.x, l.y, l.partial, l.batch, p.lpr, p.ntasks); break;
-    case 4: hipLaunchKernelGGL((gemv_kquant_kernel<FMT, 4, dual ? 2 : 4, MODE>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows, l.cols, l.x, l.y, l.partial, l.batch, p.lpr, p.ntasks); break;
-    default: hipLaunchKernelGGL((gemv_kquant_kernel<FMT, 8, dual ? 1 : 2, MODE>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows, l.cols, l.x, l.y, l.partial, l.batch, p.lpr, p.ntasks); break;
+    default: hipLaunchKernelGGL((gemv_kquant_kernel<FMT, 4, dual ? 2 : 4, MODE>), g, b, 0, s, l.w, l.w2, l.row_bytes, l.rows, l.cols, l.x, l.y, l.partial, l.batch, p.lpr, p.ntasks); break;
     }
 }
 
@@ -284,22 +282,26 @@ static int check_matrix(int fmt, const void* w, int rows, int cols) {
 // ------------------------------------------------------------ MFMA path ----
 // Whether a GGUF-row K-quant readout of `weights` values (rows x cols, both matrices of a
 // SwiGLU pair) over `batch` rows runs on the matrix cores rather than the vector ALUs.
-// Measured per call on MI355X against the vector-ALU kernel (gemv_kquant_kernel, batch
-// tiles of up to 8 rows), row layout:
-//   4096x4096 Q4_K      b2 9.5 / 19.6 us, b3 12.5 / 19.8, b4 14.3 / 20.0, b5 24.3 / 19.9
-//   12288x4096 Q4_K     b2 20.1 / 27.0, b3 27.4 / 27.3, b4 32.8 / 27.3, b5 61.2 / 27.5
-//   151936x2048 Q6_K LM head   b2 101.7 / 90.4, b4 154.5 / 90.7, b5 228.9 / 90.6,
-//                              b16 638.6 / 91.7 (vector ALUs: 135 M VALU instructions)
-//   SwiGLU MLP 2048x6144 (config 2)   b4 46.4 / 42.1, b8 78.7 / 43.8, b32 307.9 / 50.9
-// The vector path issues NB fma per weight and batch tile, so its time grows with the
-// batch; the matrix cores' does not up to 32 rows.
-constexpr int64_t kMmaAnyWeights = 0;               // from batch 5: every matrix
+// Measured per call on MI355X, GGUF rows, vector ALUs (a grid row of gemv_b1_kernel per batch
+// row) / matrix cores, us:
+//   2048x2048 Q4_K      b2 3.4 / 8.0, b4 4.1 / 8.0
+//   5003x1280 Q6_K      b2 6.8 / 11.3, b3 7.9 / 11.2, b4 9.5 / 11.3
+//   2048x6144 Q6_K      b2 10.4 / 12.5, b3 13.8 / 12.7, b4 17.2 / 12.8
+//   4096x4096 Q4_K      b2 6.4 / 9.4, b3 7.7 / 9.6, b4 9.3 / 9.5      Q6_K  b3 11.3 / 12.9, b4 14.2 / 13.0
+//   12288x4096 Q4_K     b2 14.1 / 17.3, b3 17.8 / 17.2, b4 20.9 / 17.2
+//   32000x2048 Q6_K     b2 26.4 / 24.7, b3 36.2 / 24.5
+//   151936x2048 Q6_K LM head   b2 99.6 / 82.9, b3 140.8 / 80.0
+// The vector path streams the weights once per row, the later times from the caches, so its
+// time grows with the batch; the matrix cores' does not up to 32 rows.  From 5 rows on every
+// matrix runs there (a row's result is then the same for all of 5 to 64 rows).  At batch 4 the
+// matrix cores would take over at about 12M weights; callers were told that they need no
+// workspace there (rta_gemv_workspace_bytes), so the line stays.
 constexpr int64_t kMmaMidWeights = 32ll << 20;      // from batch 3
 constexpr int64_t kMmaTallWeights = 128ll << 20;    // from batch 2
 __host__ __device__ constexpr bool mma_batch(int64_t weights, int batch) {
-    return (batch >= 5 && weights >= kMmaAnyWeights) || (batch >= 3 && weights >= kMmaMidWeights) ||
-           (batch >= 2 && weights >= kMmaTallWeights);
+    return batch >= 5 || (batch >= 3 && weights >= kMmaMidWeights) || (batch >= 2 && weights >= kMmaTallWeights);
 }
+
 struct MmaPlan {
     int nbt, total_rows, ntg, nslab, sb_per_slab, wgs_per_slab, grid;
     size_t part_bytes;

@@ -227,7 +227,11 @@ __host__ __device__ constexpr int b1_lds_bytes(int slots) { return slots * 17 * 
 
 // KW waves per row task (cols = 64*64*KW at most); 256-thread blocks run 4/KW
 // independent task groups when KW divides 4, otherwise one group of KW waves.
-// R rows per lane per task (P*R rows per task).
+// R rows per lane per task (P*R rows per task).  blockIdx.y is the batch row: batches of 2 to
+// 4 below the matrix cores' line read the weights once per row, the later times from the
+// caches (us per call against a kernel that read them once and unpacked them per x row, 2 /
+// 3 / 4 rows: 4096x4096 Q4_K 9.1 / 11.4 / 13.4 before, 6.4 / 7.7 / 9.3 so; 5003x1280 Q6_K
+// 7.5 / 10.0 / 11.8, 6.8 / 7.9 / 9.5; 2048x2048 Q4_K 7.7 / 9.9 / 11.7, 3.4 / 4.1 / 4.1).
 template <int FMT, int R, int MODE, int KW>
 __global__ void __launch_bounds__(256) gemv_b1_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                                                       const int64_t row_bytes, const int rows, const int cols,
@@ -241,6 +245,9 @@ __global__ void __launch_bounds__(256) gemv_b1_kernel(const uint8_t* __restrict_
     __shared__ float s_part[kGroups][KW][R][2][4];   // per wave partials (KW > 1), 4 subs max
     __shared__ float s_ss[4];                        // the fused RMSNorm's wave sums
 
+    x += (int64_t)blockIdx.y * cols;
+    y += (int64_t)blockIdx.y * rows;
+    if constexpr (MODE == kLogits) partial += (int64_t)blockIdx.y * ntasks;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int group = wave / KW, wk = wave - group * KW;   // wave index inside its task group
     const int S = cols >> 6, P = kWave / lpr;
@@ -393,8 +400,9 @@ __global__ void __launch_bounds__(256) gemv_b1_kernel(const uint8_t* __restrict_
     }
 }
 
-// ------------------------------------------------------------ batch > 1 ----
-// NB batch rows per launch; x slices are loaded per task (L1/L2 resident).
+// -------------------------------------------------------- very wide rows ----
+// Rows of over 16384 columns, NB batch rows per launch; x slices are loaded per task (L1/L2
+// resident).
 template <int FMT, int NB, int R, int MODE>
 __global__ void __launch_bounds__(256) gemv_kquant_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                                                           const int64_t row_bytes, const int rows, const int cols,

@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
     // x loads first (vector-memory loads complete in order, so the x slab is not held
     // up behind the weights; and a kernel starts with cold instruction and scalar
     // caches, so nothing is worked out ahead of them that they do not need), then
-    // DEPTH - 1 superblocks of weights, then the x prep.
+    // one superblock of weights, then the x prep.
     XStage<FMT, NBT> xs;
     xs.load(x, cols, batch, sb0, nsb, rn);
 

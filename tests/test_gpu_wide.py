@@ -102,3 +102,19 @@ def test_rows_of_wide_calls_do_not_depend_on_the_batch(fmt, rows, cols):
         y = {n: ops.gemv(f, wd, rows, cols, x[:n]).cpu().numpy() for n in (20, 32, 33, 64, 65, 128, 129, 257, 600)}
         for a, b in ((20, 64), (32, 33), (65, 128), (129, 600), (257, 600)):
             assert np.array_equal(y[a], y[b][:a]), (packed, a, b)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("batch", [33, 65])
+def test_step_norms_in_the_wide_readouts(packed, batch):
+    """A decode step whose readouts take the RMSNorm in front of them in their x preparation,
+    against the fp64 composition."""
+    from rta import model
+    from rta._lib import Q4_K, Q6_K
+    from step_reference import check_steps
+    t = TILED if packed else 0
+    shape = model.HybridShape(hidden=512, layers=4, full_every=2, q_heads=4, kv_heads=2, head_dim=128, rec_heads=2,
+                              ff=768, vocab=3001, capacity=64, fmt_embed=Q4_K, fmt_proj=Q4_K | t, fmt_lm=Q6_K | t,
+                              fmt_k=Q4_K, fmt_v=Q6_K, rope_rotary=128, eps=1e-6, margin=1e-4, rope_theta=1e6)
+    m = model.DecodeModel(shape, batch, [3 + 2 * i % 90 for i in range(batch)], seed=17, keep_gguf=True)
+    check_steps(m, 2)
