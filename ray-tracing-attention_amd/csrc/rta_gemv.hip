@@ -336,11 +336,15 @@ static MmaPlan plan_tiled(int rows, int cols, int nbt, bool dual) {
 }
 
 // Bytes of workspace one projection needs for its batch tiles of at most 32 rows (0 when
-// the VALU paths serve it); covers batch tiles of either width.
+// the VALU paths serve it); covers batch tiles of either width.  GGUF rows on the matrix
+// cores ask for some even where one K slab needs none: a readout that depends on the batch
+// for it is refused without one at every size, not at some.
+constexpr size_t kRowsWs = 256;
 static size_t narrow_ws(int fmt, int rows, int cols, int batch, bool dual) {
     if (!is_tiled(fmt) && !(is_kquant(fmt) && mma_batch((int64_t)rows * cols * (dual ? 2 : 1), batch))) return 0;
     const MmaPlan a = plan_tiled(rows, cols, 1, dual), b = plan_tiled(rows, cols, 2, dual);
-    return a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes;
+    const size_t part = a.part_bytes > b.part_bytes ? a.part_bytes : b.part_bytes;
+    return part || is_tiled(fmt) ? part : kRowsWs;
 }
 
 // Work split of wide_kernel (rta_wide.hpp) for a call of `batch` rows in launches of up to
@@ -529,8 +533,8 @@ static bool use_wide(int fmt, int rows, int cols, int batch, bool dual, const vo
     return need && ws && ws_bytes >= need;
 }
 
-// Runs one projection over the whole batch: K-quant tiles of >= 8 rows on the matrix
-// cores (32 rows per tile), smaller ones on the VALU kernels (8 rows per tile).
+// Runs one projection over the whole batch: K-quant tiles on the matrix cores (wide launches above
+// 32 rows, tiles of 32 below), K-quant batches under mma_batch's line and floats on the VALU kernels.
 // For kLogits, partial receives per-task maxima laid out [tile row][ntasks] inside the
 // tile's [tile x rows] region; *ntasks_out / *rows_per_task_out describe the last tile.
 template <int MODE>
@@ -572,7 +576,7 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
                                rows_per_task_out, s);
         } else if (tiled || mma) {
             const size_t need = narrow_ws(fmt, rows, cols, one_tile(whole), MODE == kSwiglu);
-            if ((!ws && (need || tiled)) || ws_bytes < need) return RTA_ERR_WORKSPACE;
+            if (!ws || ws_bytes < need) return RTA_ERR_WORKSPACE;
             e = run_tiled<MODE>(fmt, l, ws, l.partial, ntasks_out, rows_per_task_out, s);
         } else if (is_kquant(fmt)) {
             const Plan p = plan_kquant(rows, cols, chunk, MODE == kSwiglu, row_bytes);
