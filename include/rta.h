@@ -146,7 +146,8 @@ int rta_pack_remap(int fmt, const void* src, int src_rows, int cols, const rta_r
 /* SwiGLU MLP: act = sign(g) sign(u) |g| |u| sigmoid(g) with g = Wg x, u = Wu x
  * ([batch, inter]); then y (=|+=) Wd act ([batch, hidden]).
  *   Wg, Wu: [inter, hidden] (one format); Wd: [hidden, inter].
- *   Workspace: rta_mlp_workspace_bytes() (0 for batch < 8).
+ *   Workspace: rta_mlp_workspace_bytes() (0 where neither readout runs on
+ *   the matrix cores; see rta_gemv).
  * Replaces Resident::executeMLP (optical_resident.cpp:484-491): op 2 index 3
  * (resident_math.comp:54-58,71) then op 2 index 4 with the residual (:70).
  * mlpCheck (optical_resident.cpp:922-949) is epilogue STORE (state zeroed). */
