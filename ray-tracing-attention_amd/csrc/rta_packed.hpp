@@ -506,8 +506,8 @@ __global__ void __launch_bounds__(64 * NWAVES) gemm_packed_kernel(
     // wave's last unit.  One copy each of the multiplication and of finish(), the buffers
     // rotated by register moves: a kernel's code is fetched cold at every launch, and a body
     // unrolled over the two buffers with finish() three times was 24.6 KB against 13.2 (gate/up
-    // pair in the batch-32 step 22.1 -> 21.9 us; with gemm_tiled_kernel's likewise, the step
-    // 3838 -> 3776 us and a 2048-wide MLP of 8 rows 25.9 -> 23.2).
+    // pair in the batch-32 step 22.1 -> 21.9 us).  Called back to back, its code warm, that pair
+    // takes 25.2 us against 24.3: the moves cost what the step's cold starts give back.
     constexpr int kSlot = TPW * NBT * 4 * 64;   // floats per wave
     static_assert(NWAVES * kSlot * sizeof(float) <= sizeof(sx), "partial slots fit in the x images");
     float* slots = reinterpret_cast<float*>(sx);
