@@ -94,7 +94,11 @@ int rta_pack(int fmt, const void* src, int rows, int cols, void* dst, rta_stream
  *   K-quant batches of 5 or more rows (3 or more when rows x cols >= 2^25, 2 or more
  *   when >= 2^27; a SwiGLU pair counts both matrices), and packed matrices
  *   (fmt | RTA_TILED) at every batch, run on the matrix cores and need a workspace of
- *   rta_gemv_workspace_bytes() (256-byte aligned); 0 bytes otherwise.
+ *   rta_gemv_workspace_bytes() (256-byte aligned); 0 bytes otherwise.  As every size
+ *   query with a batch, it answers for all batches up to the one asked.  A K-quant or
+ *   packed call of over 32 rows also takes the workspace of 32 rows: it then runs 32 rows
+ *   at a time, reading the weights once for each, and above 64 rows it rounds differently
+ *   (other K slabs).
  * Replaces the projection detector, resident_math.comp:39-75 (op 2, indices
  * 0/1/2/4/6/8) dispatched by Resident::launch, optical_resident.cpp:304-347, and its
  * batched pipelines (optical_resident.cpp:168,343; resident_batch2.comp). */

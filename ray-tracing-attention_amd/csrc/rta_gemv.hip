@@ -406,11 +406,20 @@ static size_t wide_ws(int fmt, int rows, int cols, int batch, bool dual) {
            (p.nslab > 1 ? (size_t)p.nslab * n * (dual ? 2 : 1) * rows * sizeof(float) : 0);
 }
 
-// Workspace of a projection over `batch` rows: the narrow tiles' or the wide launches',
-// whichever is more (a caller may run a smaller batch on it).
+// Workspace of a projection over up to `batch` rows: the most that a call of 1 to `batch` rows
+// takes, by narrow tiles or wide launches.  A class's need grows with its rows, but a class of
+// fewer rows can need more than one of more rows (it is cut into more K slabs: 12288x4096
+// takes 26.3 MB for 64 rows, 12.6 MB for 65), so each class counts at its largest batch.
+// Without that a caller who allocates once for its largest batch would run the smaller ones in
+// narrow tiles, or (the decode step) be refused.
 static size_t projection_ws(int fmt, int rows, int cols, int batch, bool dual) {
-    const size_t a = narrow_ws(fmt, rows, cols, one_tile(batch), dual), b = wide_ws(fmt, rows, cols, batch, dual);
-    return a > b ? a : b;
+    size_t most = narrow_ws(fmt, rows, cols, one_tile(batch), dual);
+    for (const int top : {64, 128, batch}) {
+        const size_t need = wide_ws(fmt, rows, cols, batch < top ? batch : top, dual);
+        if (need > most) most = need;
+        if (batch <= top) break;
+    }
+    return most;
 }
 
 // The fixed-order slab reduce (gemm_reduce_kernel), its loads all in flight at once for

@@ -214,3 +214,30 @@ def test_image_readout_refusals(lib):
     assert R(ws=ctypes.c_void_p(FAKE.value + 8)) == 4
     assert R(y=FAKE_ODD) == 4
     assert R(ss=ctypes.c_void_p(FAKE.value + 4)) == 4
+
+
+def test_workspaces_of_a_larger_batch_serve_every_smaller_one(lib):
+    """A program allocates a workspace once, for its largest batch: no size query shrinks as
+    the batch grows (readouts of 33 to 64 and of 65 to 128 rows are cut into more K slabs than
+    larger ones), so a smaller batch is neither refused nor run by another path there."""
+    from rta import model
+    T = _lib.TILED
+    remap = _lib.Remap(3, 128, 64, 0)
+    queries = {}
+    for rows, cols in [(12288, 4096), (4096, 4096), (6144, 2048), (32000, 2048), (5003, 1280), (16, 256)]:
+        for f in (_lib.Q4_K, _lib.Q6_K, _lib.Q6_K | T):
+            queries["gemv", rows, cols, f] = lambda b, a=(f, rows, cols): lib.rta_gemv_workspace_bytes(*a, b)
+            queries["lm", rows, cols, f] = lambda b, a=(f, rows, cols): lib.rta_lm_head_workspace_bytes(*a, b)
+            queries["mlp", rows, cols, f] = lambda b, a=(f, f, cols, rows // 256 * 256 + 256): (
+                lib.rta_mlp_workspace_bytes(*a, b))
+    queries["remap"] = lambda b: lib.rta_gemv_remap_workspace_bytes(_lib.Q4_K, ctypes.byref(remap), 6144, 2048, b)
+    hybrid = model._lib_h()
+    step = model.HybridShape(hidden=4096, layers=4, full_every=2, q_heads=4, kv_heads=2, head_dim=128, rec_heads=2,
+                             ff=12288, vocab=300, capacity=64, fmt_embed=_lib.Q4_K, fmt_proj=_lib.Q4_K | T,
+                             fmt_lm=_lib.Q6_K | T, fmt_k=_lib.Q4_K, fmt_v=_lib.Q6_K, rope_rotary=128, eps=1e-6,
+                             margin=1e-4, rope_theta=1e6)
+    queries["step"] = lambda b: hybrid.rta_hybrid_workspace_bytes(ctypes.byref(step), b)
+    for name, query in queries.items():
+        need = [query(b) for b in [*range(1, 140), 255, 256, 257, 300, 1000]]
+        assert need[-1] > 0, name
+        assert need == sorted(need), name

@@ -105,6 +105,20 @@ def test_rows_of_wide_calls_do_not_depend_on_the_batch(fmt, rows, cols):
 
 
 @pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("rows,cols", [(6144, 2048), (1000, 4096)])
+def test_smaller_batches_on_the_largest_batchs_workspace(rows, cols, packed):
+    """Bitwise the results of a workspace of their own, where 64 rows (both shapes) and 65 to 128
+    (6144x2048) are cut into more K slabs than 256."""
+    rng = np.random.default_rng(rows + cols)
+    _, wd, f = matrix(rng, orc.Q4_K, rows, cols, packed)
+    x = dev(rng.standard_normal((256, cols)).astype(np.float32))
+    largest = dev(np.zeros(ops.gemv_workspace_bytes(f, rows, cols, 256), np.uint8))
+    for n in (20, 33, 64, 65, 100, 128, 129, 256):
+        y = ops.gemv(f, wd, rows, cols, x[:n], workspace=largest)
+        assert np.array_equal(y.cpu().numpy(), ops.gemv(f, wd, rows, cols, x[:n]).cpu().numpy()), n
+
+
+@pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("batch", [33, 65])
 def test_step_norms_in_the_wide_readouts(packed, batch):
     """A decode step whose readouts take the RMSNorm in front of them in their x preparation,
