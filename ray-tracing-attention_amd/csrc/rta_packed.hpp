@@ -502,80 +502,74 @@ __global__ void __launch_bounds__(64 * NWAVES) gemm_packed_kernel(
     const int head = cu;                      // the wave's first unit ...
     const bool head_shared = csb != 0;        // ... began in an earlier wave
     f4_t hacc[TPW][NBT];                      // its partial sums, for that wave
-    // The items, then one pass (it == nit) that hands the head partials over and closes the
-    // wave's last unit.  One copy each of the multiplication and of finish(), the buffers
-    // rotated by register moves: a kernel's code is fetched cold at every launch, and a body
-    // unrolled over the two buffers with finish() three times was 24.6 KB against 13.2 (gate/up
-    // pair in the batch-32 step 22.1 -> 21.9 us).  Called back to back, its code warm, that pair
-    // takes 25.2 us against 24.3: the moves cost what the step's cold starts give back.
-    constexpr int kSlot = TPW * NBT * 4 * 64;   // floats per wave
-    static_assert(NWAVES * kSlot * sizeof(float) <= sizeof(sx), "partial slots fit in the x images");
-    float* slots = reinterpret_cast<float*>(sx);
-#pragma clang loop unroll(disable)
-    for (int it = 0; it <= nit; ++it) {
-        bool done = false;
-        if (it < nit) {
-            load_next(nxt);
-            take_turns(wave, it);
-            compute(csb, cur);
-            if (csb == nsb - 1) {
-                if (head_shared && cu == head) {
-#pragma unroll
-                    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-                        for (int bt = 0; bt < NBT; ++bt) {
-                            hacc[t][bt] = acc[t][bt];
-                            acc[t][bt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                        }
-                } else {
-                    done = true;
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < TPW; ++t) cur[t] = nxt[t];
-        } else {
-            // units left open: the head piece of a unit that ends inside this wave's range holds
-            // only a middle part (it is the head partial), or the wave owns an unfinished unit
-            const bool open = nit > 0 && csb != 0;
-            const bool mid = open && head_shared && cu == head;
-            if (mid) {
+    const auto item = [&](int it, Raw* now, Raw* next) {
+        load_next(next);
+        take_turns(wave, it);
+        compute(csb, now);
+        if (csb == nsb - 1) {
+            if (head_shared && cu == head) {
 #pragma unroll
                 for (int t = 0; t < TPW; ++t)
 #pragma unroll
-                    for (int bt = 0; bt < NBT; ++bt) hacc[t][bt] = acc[t][bt];
-            }
-            // hand the head partials over through LDS (the x images are no longer read)
-            __syncthreads();
-            if (head_shared && nit > 0) {
-#pragma unroll
-                for (int t = 0; t < TPW; ++t)
-#pragma unroll
-                    for (int bt = 0; bt < NBT; ++bt)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            slots[wave * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane] = hacc[t][bt][e];
-            }
-            __syncthreads();
-            if (open && !mid) {   // the owner adds the pieces of the later waves in wave order
-                const int end = (cu - wa + 1) * nsb;   // items of the unit end here
-                for (int wv = wave + 1; wv < NWAVES && item0(wv) < end; ++wv) {
-                    if (item0(wv + 1) == item0(wv)) continue;   // (a wave without items holds no piece)
-#pragma unroll
-                    for (int t = 0; t < TPW; ++t)
-#pragma unroll
-                        for (int bt = 0; bt < NBT; ++bt)
-#pragma unroll
-                            for (int e = 0; e < 4; ++e)
-                                acc[t][bt][e] += slots[wv * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane];
-                }
-                done = true;
+                    for (int bt = 0; bt < NBT; ++bt) {
+                        hacc[t][bt] = acc[t][bt];
+                        acc[t][bt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                    }
+            } else {
+                finish(cu);
             }
         }
-        if (done) finish(cu);
         if (++csb == nsb) {
             csb = 0;
             ++cu;
         }
+    };
+    // Two copies of the body, the buffers changing roles.  One copy with register moves halves the
+    // code that is fetched cold at every launch, but the moves cost more (us per call, weights
+    // warm / cold, one copy -> two: gate/up 12288x4096 Q4_K of 32 rows 23.5 / 25.1 -> 23.2 / 24.3,
+    // of 1 row 16.6 / 17.6 -> 15.3 / 16.7; 10240x4096 of 32 rows 13.5 / 14.0 -> 12.7 / 13.3;
+    // 4096x12288 of 32 rows 12.4 / 12.7 -> 12.0 / 12.0).
+#pragma clang loop unroll(disable)
+    for (int it = 0; it < nit; it += 2) {
+        item(it, cur, nxt);
+        if (it + 1 < nit) item(it + 1, nxt, cur);
+    }
+    // units left open: the head piece of a unit that ends inside this wave's range holds
+    // only a middle part (it is the head partial), or the wave owns an unfinished unit
+    const bool open = nit > 0 && csb != 0;
+    const bool mid = open && head_shared && cu == head;
+    if (mid) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+            for (int bt = 0; bt < NBT; ++bt) hacc[t][bt] = acc[t][bt];
+    }
+    // hand the head partials over through LDS (the x images are no longer read)
+    constexpr int kSlot = TPW * NBT * 4 * 64;   // floats per wave
+    static_assert(NWAVES * kSlot * sizeof(float) <= sizeof(sx), "partial slots fit in the x images");
+    float* slots = reinterpret_cast<float*>(sx);
+    __syncthreads();
+    if (head_shared && nit > 0) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+            for (int bt = 0; bt < NBT; ++bt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) slots[wave * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane] = hacc[t][bt][e];
+    }
+    __syncthreads();
+    if (open && !mid) {   // the owner adds the pieces of the later waves in wave order
+        const int end = (cu - wa + 1) * nsb;   // items of the unit end here
+        for (int wv = wave + 1; wv < NWAVES && item0(wv) < end; ++wv) {
+            if (item0(wv + 1) == item0(wv)) continue;   // (a wave without items holds no piece)
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+#pragma unroll
+                for (int bt = 0; bt < NBT; ++bt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[t][bt][e] += slots[wv * kSlot + ((t * NBT + bt) * 4 + e) * 64 + lane];
+        }
+        finish(cu);
     }
 }
 
