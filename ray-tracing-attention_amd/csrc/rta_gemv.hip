@@ -804,10 +804,13 @@ int projection_store(int fmt, const void* w, int rows, int cols, const float* x,
 }
 
 // The wide readout's x preparation takes the norm where re-reading the rows once per
-// superblock costs less than a launch of its own (64 rows: 4.7 us).
+// superblock costs less than a launch of its own: up to one launch of rows.  Step of 4 layers and
+// 8000 words, norm launched / taken, us: hidden 2048 of 64 sequences 449 / 434, 256 986 / 965,
+// 512 1894 / 1895, 1024 3748 / 3768; hidden 4096 of 64 553 / 535, 256 1155 / 1138, 512
+// 2220 / 2229, 1024 4381 / 4427.
 bool wide_norm_fusable(int fmt, int rows, int cols, int batch, bool dual, size_t ws_bytes) {
     const size_t need = wide_ws(fmt, rows, cols, batch, dual);
-    return need && ws_bytes >= need && cols <= 4096;
+    return need && ws_bytes >= need && cols <= 4096 && batch <= kWideBatch;
 }
 
 bool b1_norm_fusable(int fmt, int cols, int batch) {

@@ -132,3 +132,20 @@ def test_step_norms_in_the_wide_readouts(packed, batch):
                               fmt_k=Q4_K, fmt_v=Q6_K, rope_rotary=128, eps=1e-6, margin=1e-4, rope_theta=1e6)
     m = model.DecodeModel(shape, batch, [3 + 2 * i % 90 for i in range(batch)], seed=17, keep_gguf=True)
     check_steps(m, 2)
+
+
+def small_step(hidden, batch, packed):
+    from rta import model
+    from rta._lib import Q4_K, Q6_K
+    t = TILED if packed else 0
+    shape = model.HybridShape(hidden=hidden, layers=2, full_every=2, q_heads=2, kv_heads=2, head_dim=128, rec_heads=2,
+                              ff=512, vocab=300, capacity=64, fmt_embed=Q4_K, fmt_proj=Q4_K | t, fmt_lm=Q6_K | t,
+                              fmt_k=Q4_K, fmt_v=Q6_K, rope_rotary=128, eps=1e-6, margin=1e-4, rope_theta=1e6)
+    return model.DecodeModel(shape, batch, [3 + i % 50 for i in range(batch)], seed=18, keep_gguf=True)
+
+
+@pytest.mark.parametrize("batch", [256, 257])
+def test_step_norms_at_one_launch_of_rows(batch):
+    """The readouts take the norm up to 256 sequences; above, it is a launch of its own."""
+    from step_reference import check_steps
+    check_steps(small_step(512, batch, True), 1)
