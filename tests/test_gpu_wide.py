@@ -149,3 +149,39 @@ def test_step_norms_at_one_launch_of_rows(batch):
     """The readouts take the norm up to 256 sequences; above, it is a launch of its own."""
     from step_reference import check_steps
     check_steps(small_step(512, batch, True), 1)
+
+
+@pytest.mark.parametrize("batch", [33, 257])
+def test_step_refuses_an_unaligned_norm_vector(batch):
+    """As the norm kernel itself does, also where a readout would take the norm."""
+    m = small_step(256, batch, True)
+    for name in ("norm_in", "norm_post"):
+        at = getattr(m.layers[1], name)
+        setattr(m.layers[1], name, at + 4)
+        with pytest.raises(_lib.RtaError) as e:
+            m.step()
+        assert e.value.status == 4, name
+        setattr(m.layers[1], name, at)
+    m.weights.norm_final += 4
+    with pytest.raises(_lib.RtaError) as e:
+        m.step()
+    assert e.value.status == 4
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("fmt", [orc.Q4_K, orc.Q6_K])
+@pytest.mark.parametrize("rows,cols,batch", [(130, 512, 40), (300, 768, 130), (4096, 2304, 257)])
+def test_not_finite_rows_stay_apart(fmt, packed, rows, cols, batch):
+    """Rows that hold a NaN or an infinity come out not finite, all others bit for bit as
+    without them (the same workgroup and the same matrix-core tiles hold both)."""
+    rng = np.random.default_rng(rows + batch + fmt)
+    _, wd, f = matrix(rng, fmt, rows, cols, packed)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    clean = ops.gemv(f, wd, rows, cols, dev(x)).cpu().numpy()
+    bad = {0: np.nan, 17: np.inf, 31: -np.inf, batch - 1: np.nan}
+    for b, v in bad.items():
+        x[b, (37 * b + 5) % cols] = v
+    y = ops.gemv(f, wd, rows, cols, dev(x)).cpu().numpy()
+    good = [b for b in range(batch) if b not in bad]
+    assert np.array_equal(y[good], clean[good])
+    assert not np.isfinite(y[list(bad)]).any()
