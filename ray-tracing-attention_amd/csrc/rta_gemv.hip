@@ -154,17 +154,38 @@ struct Plan {
     int nb, r, kw, lpr, ntasks, grid, block, rows_per_task;
 };
 
+// Whether 2 to 4 rows of a Q6_K matrix run faster where one wave reads a weight once for all of
+// them (gemv_kquant_kernel, `tasks` of them) than as a grid row each of the batch-1 kernel.  The
+// latter's time grows with weights times rows.  The former's grows with its rounds of a task per
+// SIMD (it is bound by its VALU work: a second wave on a SIMD takes as long again), so it wins
+// where the last round is nearly full, the more so the more rows there are, and over 4096 columns,
+// where the batch-1 kernel splits a row between waves.  us, grid row each / once for all:
+// 4000x8192 of 4 rows 32.5 / 24.0, 3906x8192 of 2 20.5 / 17.0, 3255x6144 of 4 26.8 / 22.2,
+// 16000x2048 of 4 26.2 / 23.1; but 2441x8192 of 4 (1.2 rounds) 22.7 / 22.9, 4882x4096 of 4
+// (1.2 rounds) 18.6 / 22.7, 5003x1280 of 3 8.1 / 10.1.  Over 418 sizes of 4M to 130M weights the
+// choice is 0.5% slower on the mean than the better of both, 12% at most.  Q4_K takes the grid row
+// each at every size (3906x8192 of 4 17.6 / 21.4).
+static bool q6_rows_together(int tasks, int passes, int batch) {
+    constexpr int kSimds = 4 * kPlanCUs;
+    const double fill = (double)tasks / kSimds, rounds = (double)((tasks + kSimds - 1) / kSimds);
+    const double gain = (1.05 + 0.075 * batch) * (passes > 1 ? 1.2 : 1.0);
+    return passes * rounds + 0.25 < gain * passes * fill;
+}
+
 // Launch plan of one K-quant projection over `batch` (<= 4) x rows; row_bytes of one
 // matrix row (both matrices' rows are streamed in the dual case).
-static Plan plan_kquant(int rows, int cols, int batch, bool dual, int64_t row_bytes) {
+static Plan plan_kquant(int fmt, int rows, int cols, int batch, bool dual, int64_t row_bytes) {
     Plan p{};
     const int S = cols / 64;
-    p.b1 = batch <= 4 && S <= 4 * kWave;
+    p.lpr = S >= kWave ? kWave : pow2ceil(S);
+    const int together = (kWave / p.lpr) * (dual ? 2 : 4);   // rows per task of gemv_kquant_kernel
+    const int passes = (S + kWave - 1) / kWave;
+    p.b1 = batch <= 4 && S <= 4 * kWave &&
+           !(fmt == RTA_Q6_K && batch >= 2 && q6_rows_together((rows + together - 1) / together, passes, batch));
     if (p.b1) {
         p.nb = batch;
         p.r = dual ? 1 : 2;
-        p.kw = S <= kWave ? 1 : (S + kWave - 1) / kWave;
-        p.lpr = S >= kWave ? kWave : pow2ceil(S);
+        p.kw = passes;
         p.rows_per_task = (kWave / p.lpr) * p.r;
         p.ntasks = (rows + p.rows_per_task - 1) / p.rows_per_task;
         const int groups = p.kw == 3 ? 1 : 4 / p.kw;
@@ -183,8 +204,7 @@ static Plan plan_kquant(int rows, int cols, int batch, bool dual, int64_t row_by
     p.nb = batch <= 1 ? 1 : batch <= 2 ? 2 : 4;
     p.r = dual ? 2 : 4;
     p.kw = 1;
-    p.lpr = S >= kWave ? kWave : pow2ceil(S);
-    p.rows_per_task = (kWave / p.lpr) * p.r;
+    p.rows_per_task = together;
     p.ntasks = (rows + p.rows_per_task - 1) / p.rows_per_task;
     const int wgs = (p.ntasks + 3) / 4;
     p.grid = wgs < 2048 ? wgs : 2048;
@@ -283,7 +303,7 @@ static int check_matrix(int fmt, const void* w, int rows, int cols) {
 // Whether a GGUF-row K-quant readout of `weights` values (rows x cols, both matrices of a
 // SwiGLU pair) over `batch` rows runs on the matrix cores rather than the vector ALUs.
 // Measured per call on MI355X, GGUF rows, vector ALUs (a grid row of gemv_b1_kernel per batch
-// row) / matrix cores, us:
+// row; see q6_rows_together for those of Q6_K that run otherwise) / matrix cores, us:
 //   2048x2048 Q4_K      b2 3.4 / 8.0, b4 4.1 / 8.0
 //   5003x1280 Q6_K      b2 6.8 / 11.3, b3 7.9 / 11.2, b4 9.5 / 11.3
 //   2048x6144 Q6_K      b2 10.4 / 12.5, b3 13.8 / 12.7, b4 17.2 / 12.8
@@ -588,7 +608,7 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
             if (!ws || ws_bytes < need) return RTA_ERR_WORKSPACE;
             e = run_tiled<MODE>(fmt, l, ws, l.partial, ntasks_out, rows_per_task_out, s);
         } else if (is_kquant(fmt)) {
-            const Plan p = plan_kquant(rows, cols, chunk, MODE == kSwiglu, row_bytes);
+            const Plan p = plan_kquant(fmt, rows, cols, chunk, MODE == kSwiglu, row_bytes);
             if (ntasks_out) *ntasks_out = p.ntasks;
             if (rows_per_task_out) *rows_per_task_out = p.rows_per_task;
             e = launch_kquant<MODE>(fmt, p, l, s);

@@ -227,8 +227,8 @@ __host__ __device__ constexpr int b1_lds_bytes(int slots) { return slots * 17 * 
 
 // KW waves per row task (cols = 64*64*KW at most); 256-thread blocks run 4/KW
 // independent task groups when KW divides 4, otherwise one group of KW waves.
-// R rows per lane per task (P*R rows per task).  blockIdx.y is the batch row: batches of 2 to
-// 4 below the matrix cores' line read the weights once per row, the later times from the
+// R rows per lane per task (P*R rows per task).  blockIdx.y is the batch row: most batches of 2
+// to 4 below the matrix cores' line read the weights once per row, the later times from the
 // caches (us per call against a kernel that read them once and unpacked them per x row, 2 /
 // 3 / 4 rows: 4096x4096 Q4_K 9.1 / 11.4 / 13.4 before, 6.4 / 7.7 / 9.3 so; 5003x1280 Q6_K
 // 7.5 / 10.0 / 11.8, 6.8 / 7.9 / 9.5; 2048x2048 Q4_K 7.7 / 9.9 / 11.7, 3.4 / 4.1 / 4.1).
@@ -400,9 +400,9 @@ __global__ void __launch_bounds__(256) gemv_b1_kernel(const uint8_t* __restrict_
     }
 }
 
-// -------------------------------------------------------- very wide rows ----
-// Rows of over 16384 columns, NB batch rows per launch; x slices are loaded per task (L1/L2
-// resident).
+// ---------------------------------------- very wide rows, some Q6_K batches ----
+// Rows of over 16384 columns, and 2 to 4 rows of Q6_K matrices whose tasks fill the SIMDs in
+// rounds (q6_rows_together); NB batch rows per launch, x slices loaded per task (L1/L2 resident).
 template <int FMT, int NB, int R, int MODE>
 __global__ void __launch_bounds__(256) gemv_kquant_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ w2,
                                                           const int64_t row_bytes, const int rows, const int cols,

@@ -1,6 +1,6 @@
 """GGUF-row readouts of 2 to 4 rows below the matrix cores' line: a grid row of the batch-1
-kernel per batch row, so every row is bit for bit that of a batch of 1, and (16640 columns)
-the kernel of wider rows; against the fp64 oracle, max|gpu - ref| <= 1e-5 + 1e-3 max|ref|."""
+kernel per batch row, so every row is bit for bit that of a batch of 1, or (16640 columns, some
+Q6_K matrices) one reading of the weights for all rows; against the fp64 oracle, max|gpu - ref| <= 1e-5 + 1e-3 max|ref|."""
 import numpy as np
 import pytest
 
@@ -31,6 +31,43 @@ def test_small_batches(fmt, rows, cols):
         y0 = rng.standard_normal((n, rows)).astype(np.float32)
         ya = ops.gemv(f, wd, rows, cols, dev(x[:n]), y=dev(y0), accumulate=True).cpu().numpy()
         assert np.array_equal(ya, y0 + y)
+
+
+@pytest.mark.parametrize("rows,cols", [(15100, 1024), (15200, 1024), (16369, 1024), (15361, 1280), (15401, 1280),
+                                       (3120, 6144)])
+def test_q6_rows_at_the_edge_of_full_rounds(rows, cols):
+    """Q6_K matrices either side of the line where 2 to 4 rows share one reading of the weights
+    instead of a grid row each: 15200x1024 from 4 rows, 16369x1024 from 3, 15401x1280 from 2,
+    3120x6144 (two passes a row) from 3."""
+    fmt = orc.Q6_K
+    rng = np.random.default_rng(rows + cols)
+    w, wd, f = matrix(rng, fmt, rows, cols, False, shift=2)
+    x = rng.standard_normal((4, cols)).astype(np.float32)
+    x[1] *= 1e-3
+    ref = orc.gemv_f64(fmt, w, rows, cols, x)
+    for n in (2, 3, 4):
+        y = ops.gemv(f, wd, rows, cols, dev(x[:n])).cpu().numpy()
+        for b in range(n):
+            assert_close(y[b], ref[b], f"batch {n} row {b}")
+        y0 = rng.standard_normal((n, rows)).astype(np.float32)
+        ya = ops.gemv(f, wd, rows, cols, dev(x[:n]), y=dev(y0), accumulate=True).cpu().numpy()
+        assert np.array_equal(ya, y0 + y)
+        logits, ids = ops.lm_head(f, wd, rows, cols, dev(x[:n]))
+        lg = logits.cpu().numpy()
+        assert np.array_equal(lg, y), n
+        for b in range(n):
+            assert int(ids.cpu().numpy().view(np.uint32)[b]) == orc.argmax_margin_f32(lg[b], 1e-4)
+
+
+@pytest.mark.parametrize("inter,batch", [(7424, 4), (7680, 4), (8192, 3)])
+def test_q6_swiglu_at_the_edge_of_full_rounds(inter, batch):
+    hidden, q6 = 1024, orc.Q6_K
+    rng = np.random.default_rng(inter + batch)
+    (g, gd, _), (u, ud, _) = (matrix(rng, q6, inter, hidden, False) for _ in range(2))
+    x = rng.standard_normal((batch, hidden)).astype(np.float32)
+    act = ops.swiglu(q6, gd, ud, hidden, inter, dev(x)).cpu().numpy()
+    gx, ux = (orc.gemv_f64(q6, m, inter, hidden, x) for m in (g, u))
+    assert_close(act, gx * ux / (1 + np.exp(-gx)), "activation")
 
 
 @pytest.mark.parametrize("hidden,inter,batch", [(256, 256, 2), (1280, 768, 3), (4352, 512, 4)])
