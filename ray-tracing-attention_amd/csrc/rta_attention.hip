@@ -2068,22 +2068,25 @@ __global__ void __launch_bounds__(256) full_middle_kernel(const MiddleArgs p) {
 // Combines a sequence's chunk records per query head.  A workgroup owns 128 / SPLIT of a
 // head's coordinates: groups of 32 / SPLIT threads (4 coordinates each), kAhead records in
 // flight per group.  One pass: each group folds its records into a running (m, Z, U),
-// rescaled when m grows; the groups are combined inside each wave, then across the waves
-// (the same sums as max-then-accumulate, in another order).
+// rescaled when m grows; the groups are combined at the end (the same sums as
+// max-then-accumulate, in another order).
 // Bound by latency: a handful of dependent reads of records another kernel just wrote.
 // With few (sequence, head) pairs the records per pair run to the hundreds and most compute
 // units would idle, so 512 threads take a quarter of the head each (64 records at once per
-// round of kAhead); see merge_split for the sizes.
+// round of kAhead); decode_attention_gate_stride, which launches it, has the sizes.  Their 64
+// groups are combined inside each wave first; the 8 or 16 groups of a whole head go through LDS
+// as they are (in-wave first, 64 sequences of 100 positions and 32 heads 21.5 -> 21.9 us a call).
 template <int THREADS, int SPLIT>
 __global__ void __launch_bounds__(THREADS) attn_merge_kernel(const AttnArgs a) {
     constexpr int kLanes = 32 / SPLIT, kGroups = THREADS / kLanes, kAhead = 8;
-    constexpr int kWaves = THREADS / kWave, kCols = kHd / SPLIT;
-    __shared__ float4 s_u[kWaves][kLanes];
-    __shared__ float s_zp[kWaves], s_mp[kWaves];
-    const int sh = blockIdx.x / SPLIT, part = blockIdx.x - sh * SPLIT;
+    constexpr int kCols = kHd / SPLIT;
+    constexpr int kParts = SPLIT == 1 ? kGroups : THREADS / kWave;   // combined through LDS
+    __shared__ float4 s_u[kParts][kLanes];
+    __shared__ float s_zp[kParts], s_mp[kParts];
+    const int sh = blockIdx.x / SPLIT, part = SPLIT == 1 ? 0 : blockIdx.x % SPLIT;
     const int s = sh / a.hq, h = sh - s * a.hq;
     const int tid = threadIdx.x;
-    const int grp = tid / kLanes, e = part * kLanes + tid % kLanes;
+    const int grp = threadIdx.x / kLanes, e = part * kLanes + (tid & (kLanes - 1));
     const int64_t L = a.ctx_len[s];
     const int64_t visible = L < a.capacity ? L : a.capacity;
     float* out = a.out + (int64_t)sh * kHd;
@@ -2158,42 +2161,45 @@ __global__ void __launch_bounds__(THREADS) attn_merge_kernel(const AttnArgs a) {
             }
         }
     }
-    // combine the groups of a wave (every lane ends with its wave's sums)
+    if constexpr (SPLIT > 1) {
+        // combine the groups of a wave (every lane ends with its wave's sums)
 #pragma unroll
-    for (int off = kLanes; off < kWave; off <<= 1) {
-        const float M2 = __shfl_xor(Mg, off, kWave), Z2 = __shfl_xor(Z, off, kWave);
-        const float4 U2 = make_float4(__shfl_xor(U.x, off, kWave), __shfl_xor(U.y, off, kWave),
-                                      __shfl_xor(U.z, off, kWave), __shfl_xor(U.w, off, kWave));
-        const float M = fmaxf(Mg, M2);
-        const float f = Mg == -INFINITY ? 0.0f : expf(Mg - M), f2 = M2 == -INFINITY ? 0.0f : expf(M2 - M);
-        Z = fmaf(Z, f, Z2 * f2);
-        U.x = fmaf(U.x, f, U2.x * f2);
-        U.y = fmaf(U.y, f, U2.y * f2);
-        U.z = fmaf(U.z, f, U2.z * f2);
-        U.w = fmaf(U.w, f, U2.w * f2);
-        Mg = M;
+        for (int off = kLanes; off < kWave; off <<= 1) {
+            const float M2 = __shfl_xor(Mg, off, kWave), Z2 = __shfl_xor(Z, off, kWave);
+            const float4 U2 = make_float4(__shfl_xor(U.x, off, kWave), __shfl_xor(U.y, off, kWave),
+                                          __shfl_xor(U.z, off, kWave), __shfl_xor(U.w, off, kWave));
+            const float M = fmaxf(Mg, M2);
+            const float f = Mg == -INFINITY ? 0.0f : expf(Mg - M), f2 = M2 == -INFINITY ? 0.0f : expf(M2 - M);
+            Z = fmaf(Z, f, Z2 * f2);
+            U.x = fmaf(U.x, f, U2.x * f2);
+            U.y = fmaf(U.y, f, U2.y * f2);
+            U.z = fmaf(U.z, f, U2.z * f2);
+            U.w = fmaf(U.w, f, U2.w * f2);
+            Mg = M;
+        }
     }
-    const int wave = tid >> 6;
-    if ((tid & 63) < kLanes) s_u[wave][tid & 63] = U;
-    if ((tid & 63) == 0) {
-        s_zp[wave] = Z;
-        s_mp[wave] = Mg;
+    constexpr int kPart = THREADS / kParts;   // threads of a part
+    const int p = tid / kPart, pl = tid & (kPart - 1);
+    if (kPart == kLanes || pl < kLanes) s_u[p][pl] = U;
+    if (pl == 0) {
+        s_zp[p] = Z;
+        s_mp[p] = Mg;
     }
     __syncthreads();
     if (tid < kCols) {
         const int c = part * kCols + tid;   // coordinate of the head
         float M = -INFINITY;
 #pragma unroll
-        for (int g = 0; g < kWaves; ++g) M = fmaxf(M, s_mp[g]);
+        for (int g = 0; g < kParts; ++g) M = fmaxf(M, s_mp[g]);
         float u = 0.0f, z = 0.0f;
 #pragma unroll
-        for (int g = 0; g < kWaves; ++g) {
+        for (int g = 0; g < kParts; ++g) {
             const float f = s_mp[g] == -INFINITY ? 0.0f : expf(s_mp[g] - M);
             u = fmaf(reinterpret_cast<const float*>(&s_u[g][0])[tid], f, u);
             z = fmaf(s_zp[g], f, z);
         }
         float o = u / fmaxf(z, 1e-30f);
-        if (a.gate) o *= detector_sigmoid(a.gate[(int64_t)s * a.gate_stride + h * kHd + c]);
+        if (a.gate) o *= detector_sigmoid(a.gate[(int64_t)(sh / a.hq) * a.gate_stride + (sh % a.hq) * kHd + c]);
         // with out_rotary R the head's rotary-pair order goes back to the exporter's
         // half-split column order (originalRotaryAxis), the columns the O projection's
         // axis remap reads (resident_quant.glsl:20,25)
