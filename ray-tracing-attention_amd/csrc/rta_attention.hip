@@ -357,25 +357,22 @@ __device__ __forceinline__ void attn_plan_wave(const AttnArgs& a) {
         scan(t, before, total);
         if (s < a.nseq) a.plan[s] = (int32_t)(carry + before);
         // The run of workgroups whose first tile lies in each sequence: short runs by the
-        // sequence's own lane, runs much longer than the sequences are many by the whole wave,
-        // sequence by sequence.  One lane alone took 16.2 us for a sequence of 512 workgroups,
-        // the wave 4.7 (launch included); 27 sequences of 2 workgroups the other way round,
-        // 2 us more for the call
+        // sequence's own lane, each long one by the whole wave.  A lane takes ~32 ns an entry (one
+        // sequence of 512 workgroups 16.2 us, 4.7 by the wave, launch included), the wave ~70 ns a
+        // run; at a line of 32 neither side can take much over 1 us for 512 workgroups
         const int64_t first = carry + before, end = first + t;
         int w0 = 0, w1 = 0;   // at most nwg workgroups
         if (t > 0) {
             w0 = (int)((first * P + T - 1) / T);
             w1 = (int)((end * P + T - 1) / T);
         }
-        const int here = a.nseq - s0 < kWave ? a.nseq - s0 : kWave;
-        if (__builtin_amdgcn_ballot_w64(w1 - w0 > 4 * here) == 0) {
+        constexpr int kShort = 32;
+        uint64_t wide = __builtin_amdgcn_ballot_w64(w1 - w0 > kShort);
+        if (w1 - w0 <= kShort)
             for (int w = w0; w < w1; ++w) a.plan[a.nseq + 1 + w] = s;
-        } else {
-            for (int i = 0; i < here; ++i) {   // uniform
-                const int wb = __builtin_amdgcn_readlane(w1, i);
-                for (int w = __builtin_amdgcn_readlane(w0, i) + lane; w < wb; w += kWave)
-                    a.plan[a.nseq + 1 + w] = s0 + i;
-            }
+        for (; wide; wide &= wide - 1) {   // uniform
+            const int i = __builtin_ctzll(wide), wb = __builtin_amdgcn_readlane(w1, i);
+            for (int w = __builtin_amdgcn_readlane(w0, i) + lane; w < wb; w += kWave) a.plan[a.nseq + 1 + w] = s0 + i;
         }
         carry += total;
     }

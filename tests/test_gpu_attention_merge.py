@@ -24,3 +24,13 @@ def test_tile_list_of_70_uneven_sequences(torch_dev):  # noqa: F811
     ctx = np.full(70, 3)
     ctx[[0, 5, 63, 64, 69]] = [6000, 64, 12000, 65, 9000]
     _sized_case(torch, dev, 72, ctx, 8, 2, (orc.Q4_K, orc.Q6_K))
+
+
+@pytest.mark.parametrize("nseq", [4, 64, 66])
+def test_tile_list_at_the_line_of_long_runs(torch_dev, nseq):  # noqa: F811
+    """Runs of 31 to 33 workgroups and of none, side by side: up to 32 are listed by the
+    sequence's own lane, longer ones by the wave."""
+    torch, dev = torch_dev
+    ctx = np.full(nseq, 1)
+    ctx[[0, 1, 2, nseq - 1]] = [2048, 2112, 1984, 2112]
+    _sized_case(torch, dev, 73 + nseq, ctx, 8, 2, (orc.Q4_K, orc.Q6_K))
