@@ -359,16 +359,32 @@ def w_mlp(torch, args, orc):
     return res
 
 
+def q6_rows_together(rows, cols, batch, pair):
+    """The library's rule for 2 to 4 rows of a Q6_K matrix: one reading of the weights for all
+    of them where its tasks nearly fill their last round of a task per SIMD."""
+    slots = cols // 64
+    lanes = 64 if slots >= 64 else 1 << (slots - 1).bit_length()
+    per_task = 64 // lanes * (2 if pair else 4)
+    tasks, passes = -(-rows // per_task), -(-slots // 64)
+    gain = (1.05 + 0.075 * batch) * (1.2 if passes > 1 else 1.0)
+    return passes * -(-tasks // 1024) + 0.25 < gain * passes * tasks / 1024
+
+
 def readout_name(fmt_name, rows, cols, batch, packed, pair=False):
     """The kernel a projection readout runs (the library's dispatch, for the bench line's
-    label): packed tiles on the matrix cores; GGUF rows on the vector-ALU
-    readout, or the matrix cores from batch 5 (3 at 2^25+ weights, 2 at
+    label): over 32 rows the wide readout; packed tiles on the matrix cores; GGUF rows on the
+    vector-ALU readouts, or the matrix cores from batch 5 (3 at 2^25+ weights, 2 at
     2^27+ weights, a SwiGLU pair counting both matrices)."""
+    if batch > 32:
+        return (f"wide_xprep_kernel<{fmt_name}> + wide_kernel<{fmt_name}> "
+                f"({'packed tiles' if packed else 'GGUF rows'}, matrix cores)")
     if packed:
         return f"gemm_tiled_kernel<{fmt_name}> (packed tiles, matrix cores)"
     weights = rows * cols * (2 if pair else 1)
     if batch >= 5 or (batch >= 3 and weights >= 1 << 25) or (batch >= 2 and weights >= 1 << 27):
         return f"gemm_tiled_kernel<{fmt_name}> (GGUF rows, matrix cores)"
+    if cols > 16384 or (fmt_name == "Q6_K" and batch >= 2 and q6_rows_together(rows, cols, batch, pair)):
+        return f"gemv_kquant_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
     return f"gemv_b1_kernel<{fmt_name}> (GGUF rows, vector ALUs)"
 
 

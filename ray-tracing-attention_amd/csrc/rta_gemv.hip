@@ -302,20 +302,29 @@ static int check_matrix(int fmt, const void* w, int rows, int cols) {
 // ------------------------------------------------------------ MFMA path ----
 // Whether a GGUF-row K-quant readout of `weights` values (rows x cols, both matrices of a
 // SwiGLU pair) over `batch` rows runs on the matrix cores rather than the vector ALUs.
-// Measured per call on MI355X, GGUF rows, vector ALUs (a grid row of gemv_b1_kernel per batch
-// row; see q6_rows_together for those of Q6_K that run otherwise) / matrix cores, us:
-//   2048x2048 Q4_K      b2 3.4 / 8.0, b4 4.1 / 8.0
-//   5003x1280 Q6_K      b2 6.8 / 11.3, b3 7.9 / 11.2, b4 9.5 / 11.3
-//   2048x6144 Q6_K      b2 10.4 / 12.5, b3 13.8 / 12.7, b4 17.2 / 12.8
-//   4096x4096 Q4_K      b2 6.4 / 9.4, b3 7.7 / 9.6, b4 9.3 / 9.5      Q6_K  b3 11.3 / 12.9, b4 14.2 / 13.0
-//   12288x4096 Q4_K     b2 14.1 / 17.3, b3 17.8 / 17.2, b4 20.9 / 17.2
-//   32000x2048 Q6_K     b2 26.4 / 24.7, b3 36.2 / 24.5
-//   151936x2048 Q6_K LM head   b2 99.6 / 82.9, b3 140.8 / 80.0
+// us per call on MI355X, GGUF rows rotating through 700 MB, vector ALUs (a grid row of
+// gemv_b1_kernel per batch row; see q6_rows_together for those of Q6_K that run otherwise) /
+// matrix cores:
+//                       2 rows      3           4           5           8           16
+//   2048x2048 Q4_K      3.7 / 8.1   4.3 / 8.1   4.4 / 8.1   4.9 / 8.1   6.2 / 8.1   9.3 / 8.2
+//   5003x1280 Q4_K      5.0 / 8.3   6.1 / 8.3   6.8 / 8.4   8.5 / 8.4  11.1 / 8.5  18.7 / 8.7
+//   4096x4096 Q4_K      6.4 / 8.9   7.6 / 8.9   9.2 / 8.9  10.8 / 9.0  15.2 / 9.1  26.7 / 9.5
+//   12288x4096 Q4_K    14.3 / 17.0 17.7 / 16.8 21.1 / 16.9 25.1 / 17.0 36.0 / 17.6
+//   2048x2048 Q6_K      4.2 / 11.0  5.1 / 11.2  5.2 / 11.2  7.1 / 11.3  8.4 / 11.3 14.4 / 11.3
+//   5003x1280 Q6_K      7.0 / 11.3  8.3 / 11.4 10.0 / 11.4 12.7 / 11.5 17.2 / 11.6
+//   2048x6144 Q6_K     10.9 / 12.5 14.2 / 12.5 17.5 / 12.5 21.2 / 12.5 31.2 / 12.5
+//   32000x2048 Q6_K    28.1 / 25.0 36.7 / 24.3 45.5 / 24.4
+//   SwiGLU 512 -> 1536 Q4_K      3.4 / 7.3   3.4 / 7.4   3.4 / 7.4   3.5 / 7.5   4.2 / 7.5   4.9 / 7.6
+//   SwiGLU 2048 -> 6144 Q4_K     8.4 / 11.1 10.8 / 11.1 13.1 / 11.2 15.2 / 11.3 22.1 / 11.8
+//   SwiGLU 2048 -> 6144 Q6_K    13.0 / 14.7 18.0 / 14.9 21.7 / 15.0 25.5 / 15.1 38.2 / 15.9
 // The vector path streams the weights once per row, the later times from the caches, so its
-// time grows with the batch; the matrix cores' does not up to 32 rows.  From 5 rows on every
-// matrix runs there (a row's result is then the same for all of 5 to 64 rows).  At batch 4 the
-// matrix cores would take over at about 12M weights; callers were told that they need no
-// workspace there (rta_gemv_workspace_bytes), so the line stays.
+// time grows with the batch; the matrix cores' does not up to 32 rows.  The lines are older than
+// the grid rows and are not where these two kernels cross: at 3 and 4 rows the matrix cores are
+// ahead from about 12M weights, and up to about 4M weights the vector ALUs to about 12 rows.  They
+// stay because a call below them has been told that it needs no workspace
+// (rta_gemv_workspace_bytes answers 0), and the path of a call does not depend on whether one
+// comes all the same; and because from 5 rows on a row's result is the same for all of 5 to 16
+// rows, and for all of 17 to 64 (other K slabs).
 constexpr int64_t kMmaMidWeights = 32ll << 20;      // from batch 3
 constexpr int64_t kMmaTallWeights = 128ll << 20;    // from batch 2
 __host__ __device__ constexpr bool mma_batch(int64_t weights, int batch) {
@@ -371,7 +380,11 @@ static size_t narrow_ws(int fmt, int rows, int cols, int batch, bool dual) {
 // kWideBatch: the tile width and K slabs with the least estimated time.  One workgroup per
 // compute unit at a time; per superblock 17 MFMAs x 2 waves per SIMD for each of its TN x NB
 // tiles, a start of a few microseconds, and for K slabs the partials' trip through memory
-// and the reduce.  The plan follows the batch's class (64, 128, more) and not the batch, so
+// and the reduce.  Against every pair of the two over 9 matrices of 2.9M to 100M weights and 128
+// and 256 rows (packed Q4_K), the estimate's choice was within 3% of the best at 10 of the 18,
+// 7 to 14% slower at 4 (12288x4096 of 256 rows 69.0 us, 63.2 with 6 tiles and 2 slabs) and 20 to
+// 33% at 4 (SwiGLU 2048 -> 6144 of 128 rows 37.6, 28.2 with 6 and 4): it is too shy of slabs for
+// wide matrices of few superblocks.  The plan follows the batch's class (64, 128, more) and not the batch, so
 // that a row's result does not depend on the rows beside it; up to 64 rows take the narrow
 // tiles' slabs (see kWideSplit).
 constexpr double kWideStartUs = 4.0, kWideTileUs = 0.2267, kWideReduceUs = 3.0, kWidePartUs = 2e-6;
@@ -575,8 +588,8 @@ static int run_projection(int fmt, const void* w, const void* w2, int rows, int 
     const bool tiled = is_tiled(fmt);
     const int64_t row_bytes = tiled ? 0 : host::row_bytes(fmt, cols);
     int b0 = 0;
-    // The path depends on the whole batch (and the matrix), so a row's result never
-    // depends on tiling.
+    // The path depends on the whole batch and the matrix (above 32 rows also on whether the
+    // workspace holds the wide launches'), so a row's result never depends on tiling.
     const bool mma = is_kquant(fmt) &&
                      mma_batch((int64_t)rows * cols * (MODE == kSwiglu ? 2 : 1), path_batch > 0 ? path_batch : batch);
     const int whole = path_batch > 0 ? path_batch : batch;

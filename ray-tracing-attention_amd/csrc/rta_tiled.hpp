@@ -202,11 +202,6 @@ __device__ __forceinline__ uint32_t word_of(const uint4& v, int i) {
     return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w;
 }
 
-// Scales and minima of groups 2 s and 2 s + 1 from a packed Q4_K tile row header h (the
-// regrouped field of TileFmt<RTA_Q4_K>): the words holding segment s's 24 bits are
-// picked with the lane's masks (bit selects: an indexed pick among the header's words
-// would go through memory), one funnel shift brings the bits down, four field extracts
-// split them.
 // Waves w and w + 4 of an 8-wave workgroup share a SIMD, whose arbiter issues for the
 // older wave first: left to it, the older wave finishes its items ~3 us before the
 // younger one, which then runs alone on the SIMD.  The two take turns at the higher
@@ -223,6 +218,11 @@ struct Q4kSegment {
     __device__ explicit Q4kSegment(int s)
         : m01(s < 2 ? ~0u : 0u), m2(s == 2 ? ~0u : 0u), shift((uint32_t)(24 * s) & 31u) {}
 };
+// Scales and minima of groups 2 s and 2 s + 1 from a packed Q4_K tile row header h (the
+// regrouped field of TileFmt<RTA_Q4_K>): the words holding segment s's 24 bits are
+// picked with the lane's masks (bit selects: an indexed pick among the header's words
+// would go through memory), one funnel shift brings the bits down, four field extracts
+// split them.
 __device__ __forceinline__ void q4k_tile_scale_min(const uint4& h, const Q4kSegment& g, uint32_t& sc0, uint32_t& sc1,
                                                    uint32_t& m0, uint32_t& m1) {
     const uint32_t w23 = (h.z & g.m2) | (h.w & ~g.m2);      // segment 2: z, segment 3: w
@@ -508,7 +508,6 @@ __global__ void __launch_bounds__(64 * kGemmWaves) gemm_tiled_kernel(
 #pragma unroll
         for (int bt = 0; bt < NBT; ++bt) acc[t][bt] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // One superblock of the unit's tiles (the second only when has2).
     // One superblock of the unit's two tiles.  Both tiles are always multiplied (at an
     // odd end of the wave's range the second repeats the first and finish() skips it),
     // so the loop body has no branches and the x operands of the next column offset

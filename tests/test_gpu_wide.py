@@ -185,3 +185,21 @@ def test_not_finite_rows_stay_apart(fmt, packed, rows, cols, batch):
     good = [b for b in range(batch) if b not in bad]
     assert np.array_equal(y[good], clean[good])
     assert not np.isfinite(y[list(bad)]).any()
+
+
+@pytest.mark.parametrize("fmt", [orc.Q4_K, orc.Q6_K])
+@pytest.mark.parametrize("rows,cols", [(700, 4096), (20000, 2304)])
+def test_rows_of_matrix_core_calls_do_not_depend_on_the_batch(fmt, rows, cols):
+    """Bitwise within 5 to 16 rows and within 17 to 64 (20000x2304: 3 K slabs of the one class,
+    5 of the other), on packed tiles and GGUF rows, which give each other's results too."""
+    rng = np.random.default_rng(rows + cols + fmt)
+    x = dev(rng.standard_normal((64, cols)).astype(np.float32))
+    both = []
+    w = synth.random_matrix(rng, fmt, rows, cols)
+    for wd, f in ((dev(w.reshape(-1)), fmt), (ops.pack(fmt, dev(w), rows, cols), fmt | TILED)):
+        y = {n: ops.gemv(f, wd, rows, cols, x[:n]).cpu().numpy() for n in (5, 11, 16, 17, 32, 64)}
+        for a, b in ((5, 16), (11, 16), (17, 32), (17, 64)):
+            assert np.array_equal(y[a], y[b][:a]), (f, a, b)
+        both.append(y)
+    for n in both[0]:
+        assert np.array_equal(both[0][n], both[1][n]), n
