@@ -533,7 +533,8 @@ def w_proj(torch, args, orc):
         ops.gemv(kfmt, copies[i % len(copies)], rows, cols, xd, y=y, workspace=ws)
 
     alg = w.nbytes + batch * 4 * (cols + rows)
-    res = {"alg_bytes": alg, "kernel": "dequant-fused projection (matrix cores from batch 5; 3 at 2^25+ weights, 2 at 2^27+)", "step": step,
+    res = {"alg_bytes": alg, "kernel": "projection readout: " + readout_name(args.fmt.upper().replace("K", "_K"), rows, cols, batch, args.packed),
+           "step": step,
            "kernel_launch": step, "unit": "GB/s", "value_from_ms": lambda ms: alg / (ms * 1e-3) / 1e9,
            "dtype": f"{args.fmt} weights x fp32 activations, fp32 accumulate",
            "config": {"workload": f"{args.fmt.upper()} projection {rows}x{cols}, batch {batch}"
@@ -860,7 +861,8 @@ def main():
     else:
         k_mean = time_kernel(torch, wl["kernel_launch"])
         kernel_name, alg_k = wl["kernel"], wl.get("alg_bytes_kernel", wl["alg_bytes"])
-        traffic = traffic_for(args.workload)
+        # counted for GGUF rows at the workload's default batch
+        traffic = traffic_for(args.workload) if not args.packed and args.batch in (None, 1) else None
     achieved = alg_k / (k_mean * 1e-3) / 1e9
     cpu = None if (args.no_cpu or wl["cpu"] is None) else wl["cpu"](args.cpu_seconds)
     line = {"metric": METRIC, "value": wl["value_from_ms"](ms_step), "unit": wl["unit"], "n_gpus": 1,
