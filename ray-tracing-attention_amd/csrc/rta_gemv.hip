@@ -439,16 +439,21 @@ static size_t wide_ws(int fmt, int rows, int cols, int batch, bool dual) {
            (p.nslab > 1 ? (size_t)p.nslab * n * (dual ? 2 : 1) * rows * sizeof(float) : 0);
 }
 
-// Workspace of a projection over up to `batch` rows: the most that a call of 1 to `batch` rows
-// takes, by narrow tiles or wide launches.  A class's need grows with its rows, but a class of
-// fewer rows can need more than one of more rows (it is cut into more K slabs: 12288x4096
-// takes 26.3 MB for 64 rows, 12.6 MB for 65), so each class counts at its largest batch.
-// Without that a caller who allocates once for its largest batch would run the smaller ones in
-// narrow tiles, or (the decode step) be refused.
+// Workspace a projection over exactly `batch` rows takes, by narrow tiles or wide launches.
+static size_t exact_ws(int fmt, int rows, int cols, int batch, bool dual) {
+    const size_t a = narrow_ws(fmt, rows, cols, one_tile(batch), dual), b = wide_ws(fmt, rows, cols, batch, dual);
+    return a > b ? a : b;
+}
+
+// ... and over up to `batch` rows, which the size queries answer.  A class's need grows with its
+// rows, but a class of fewer rows can need more than one of more rows (it is cut into more K slabs:
+// 12288x4096 takes 26.3 MB for 64 rows, 12.6 MB for 65), so each class counts at its largest
+// batch.  Without that a caller who allocates once for its largest batch would run the smaller
+// ones in narrow tiles, or (the decode step) be refused.
 static size_t projection_ws(int fmt, int rows, int cols, int batch, bool dual) {
-    size_t most = narrow_ws(fmt, rows, cols, one_tile(batch), dual);
+    size_t most = 0;
     for (const int top : {64, 128, batch}) {
-        const size_t need = wide_ws(fmt, rows, cols, batch < top ? batch : top, dual);
+        const size_t need = exact_ws(fmt, rows, cols, batch < top ? batch : top, dual);
         if (need > most) most = need;
         if (batch <= top) break;
     }
@@ -836,6 +841,11 @@ int projection_store(int fmt, const void* w, int rows, int cols, const float* x,
                                   0, rn, xn);
 }
 
+size_t readout_ws_bytes(int fmt, int rows, int cols, int batch, bool dual, bool upto) {
+    if (rows <= 0 || cols <= 0 || batch <= 0 || ((is_kquant(fmt) || is_tiled(fmt)) && cols % 256)) return 0;
+    return upto ? projection_ws(fmt, rows, cols, batch, dual) : exact_ws(fmt, rows, cols, batch, dual);
+}
+
 // The wide readout's x preparation takes the norm where re-reading the rows once per
 // superblock costs less than a launch of its own: up to one launch of rows.  Step of 4 layers and
 // 8000 words, norm launched / taken, us: hidden 2048 of 64 sequences 449 / 434, 256 986 / 965,
@@ -934,8 +944,7 @@ int rta_dequant(int fmt, const void* src, int64_t n, float* out, rta_stream_t st
 }
 
 size_t rta_gemv_workspace_bytes(int fmt, int rows, int cols, int batch) {
-    if (rows <= 0 || cols <= 0 || batch <= 0 || ((is_kquant(fmt) || is_tiled(fmt)) && cols % 256)) return 0;
-    return projection_ws(fmt, rows, cols, batch, false);
+    return readout_ws_bytes(fmt, rows, cols, batch, false, true);
 }
 
 int rta_gemv(int fmt, const void* w, int rows, int cols, const float* x, int batch, float* y, int epilogue,

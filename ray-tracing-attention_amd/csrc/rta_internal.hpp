@@ -30,6 +30,10 @@ bool b1_norm_fusable(int fmt, int cols, int batch);
 // workspace the call will pass).
 bool wide_norm_fusable(int fmt, int rows, int cols, int batch, bool dual, size_t ws_bytes);
 
+// The workspace a readout (dual: of a SwiGLU pair) over exactly `batch` rows takes, or (upto)
+// the most that one of up to `batch` rows takes, which the size queries answer.
+size_t readout_ws_bytes(int fmt, int rows, int cols, int batch, bool dual, bool upto);
+
 // y = W x (rta_gemv with the STORE epilogue) with a deferred RMSNorm factor (rn) or the
 // batch-1 readout's own RMSNorm (xn).
 int projection_store(int fmt, const void* w, int rows, int cols, const float* x, int batch, float* y, void* ws,

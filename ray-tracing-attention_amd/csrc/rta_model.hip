@@ -153,15 +153,23 @@ struct Work {
     size_t attn_bytes, lm_bytes, gemm_bytes;
 };
 
+// The sizes below are those of a step of exactly B sequences, which the step lays its workspace
+// out by, or (upto) of every batch up to B, which the size query answers.
+size_t lm_ws_bytes(int f, int V, int D, int B, bool upto) {
+    const size_t most = rta_lm_head_workspace_bytes(f, V, D, B);
+    if (upto || !most) return most;
+    return (((size_t)V * B * sizeof(float) + 255) & ~(size_t)255) + readout_ws_bytes(f, V, D, B, false, false);
+}
+
 // The largest projection workspace of an in-projection part: parts may have any row
 // count up to the whole in-projection's, and a readout's workspace does not grow steadily
 // with its rows (fewer row tiles get more K slabs).  Within one run of row counts that
 // share a plan (the same number of 16- or 32-row tiles) the slab partials grow with the
-// rows, so the multiples of 16 bound every count.  Cached per (hidden, batch, rows).
-size_t parts_ws_bytes(int D, int B, int rows_max) {
+// rows, so the multiples of 16 bound every count.  Cached per its arguments.
+size_t parts_ws_bytes(int D, int B, int rows_max, bool upto) {
     static std::mutex mu;
-    static std::map<std::tuple<int, int, int>, size_t> memo;
-    const auto key = std::make_tuple(D, B, rows_max);
+    static std::map<std::tuple<int, int, int, bool>, size_t> memo;
+    const auto key = std::make_tuple(D, B, rows_max, upto);
     {
         std::lock_guard<std::mutex> g(mu);
         const auto it = memo.find(key);
@@ -169,7 +177,7 @@ size_t parts_ws_bytes(int D, int B, int rows_max) {
     }
     size_t m = 0;
     for (const int f : {(int)RTA_Q4_K, (int)RTA_Q6_K, RTA_Q4_K | RTA_TILED, RTA_Q6_K | RTA_TILED})
-        for (int n = 16; n < rows_max + 16; n += 16) m = std::max(m, rta_gemv_workspace_bytes(f, n, D, B));
+        for (int n = 16; n < rows_max + 16; n += 16) m = std::max(m, readout_ws_bytes(f, n, D, B, false, upto));
     std::lock_guard<std::mutex> g(mu);
     memo[key] = m;
     return m;
@@ -177,36 +185,40 @@ size_t parts_ws_bytes(int D, int B, int rows_max) {
 
 // The projection workspace: enough for every format a layer may use (the shape alone
 // fixes the size), the K-quant and packed ones being the only that need any.
-size_t gemm_ws_bytes(const rta_hybrid_shape* s, const Dims& d) {
+size_t gemm_ws_bytes(const rta_hybrid_shape* s, const Dims& d, bool upto) {
     size_t m = 0;
     auto up = [&](size_t v) { m = std::max(m, v); };
+    auto need = [&](int f, int rows, int cols, bool dual = false) {
+        return readout_ws_bytes(f, rows, cols, d.B, dual, upto);
+    };
     const int fmts[5] = {s->fmt_proj, RTA_Q4_K, RTA_Q6_K, RTA_Q4_K | RTA_TILED, RTA_Q6_K | RTA_TILED};
     for (int i = s->layer_formats ? 0 : 4; i < 5; ++i) {
         const int f = s->layer_formats ? fmts[i] : s->fmt_proj;
-        if (d.nfull) up(rta_gemv_workspace_bytes(f, d.rows_full, d.D, d.B));
-        if (d.nrec) up(rta_gemv_workspace_bytes(f, d.rows_rec, d.D, d.B));
-        if (d.nrec) up(rta_gemv_workspace_bytes(f, d.H, d.D, d.B));
-        if (d.nfull) up(rta_gemv_workspace_bytes(f, d.D, d.hq * d.hd, d.B));
-        if (d.nrec) up(rta_gemv_workspace_bytes(f, d.D, d.S, d.B));
-        up(rta_mlp_workspace_bytes(f, f, d.D, d.FF, d.B));
+        if (d.nfull) up(need(f, d.rows_full, d.D));
+        if (d.nrec) up(need(f, d.rows_rec, d.D));
+        if (d.nrec) up(need(f, d.H, d.D));
+        if (d.nfull) up(need(f, d.D, d.hq * d.hd));
+        if (d.nrec) up(need(f, d.D, d.S));
+        up(need(f, d.FF, d.D, true));
+        up(need(f, d.D, d.FF));
     }
     if (d.nfull) up(image_readout_ws_bytes(d.rows_full, d.D, false));
     if (d.nrec) up(image_readout_ws_bytes(d.rows_rec, d.D, false));
     up(image_readout_ws_bytes(d.FF, d.D, true));
     up(image_readout_ws_bytes(d.D, d.FF, false));
     if (s->layer_formats)   // in-projection parts of any row count (they need layer formats)
-        up(parts_ws_bytes(d.D, d.B, std::max(d.nfull ? d.rows_full : 0, d.nrec ? d.rows_rec : 0)));
+        up(parts_ws_bytes(d.D, d.B, std::max(d.nfull ? d.rows_full : 0, d.nrec ? d.rows_rec : 0), upto));
     if (d.nrec && s->layer_formats) {   // separate a / b readouts behind a layer's pending K slabs
         size_t ab = 0;
-        for (int f : {RTA_Q4_K, RTA_Q6_K}) ab = std::max(ab, rta_gemv_workspace_bytes(f, d.H, d.D, d.B));
+        for (int f : {RTA_Q4_K, RTA_Q6_K}) ab = std::max(ab, need(f, d.H, d.D));
         const size_t slabs = std::max(image_readout_ws_bytes(d.rows_rec, d.D, false),
-                                      rta_gemv_workspace_bytes(RTA_Q6_K | RTA_TILED, d.rows_rec, d.D, d.B));
+                                      need(RTA_Q6_K | RTA_TILED, d.rows_rec, d.D));
         up(((slabs + 255) & ~(size_t)255) + ab);
     }
     return m;
 }
 
-Work carve_work(const rta_hybrid_shape* s, const Dims& d, void* p, size_t* bytes) {
+Work carve_work(const rta_hybrid_shape* s, const Dims& d, void* p, size_t* bytes, bool upto) {
     Carve c(p);
     Work w{};
     const size_t B = d.B;
@@ -227,9 +239,9 @@ Work carve_work(const rta_hybrid_shape* s, const Dims& d, void* p, size_t* bytes
     w.visible = c.take<int32_t>(B);
     w.attn_bytes = d.nfull ? rta_decode_attention_workspace_bytes(d.B, d.hq, d.hkv, d.hd, d.cap) : 0;
     w.attn_ws = c.take<uint8_t>(std::max<size_t>(w.attn_bytes, 1));
-    w.lm_bytes = rta_lm_head_workspace_bytes(s->fmt_lm, d.V, d.D, d.B);
+    w.lm_bytes = lm_ws_bytes(s->fmt_lm, d.V, d.D, d.B, upto);
     w.lm_ws = c.take<uint8_t>(std::max<size_t>(w.lm_bytes, 1));
-    w.gemm_bytes = gemm_ws_bytes(s, d);
+    w.gemm_bytes = gemm_ws_bytes(s, d, upto);
     w.gemm_ws = c.take<uint8_t>(std::max<size_t>(w.gemm_bytes, 1));
     // x images: in front of the in-projections and gate/up (D columns) and of the down
     // projection (FF columns), one at a time
@@ -256,7 +268,7 @@ size_t rta_hybrid_state_bytes(const rta_hybrid_shape* shape, int batch) {
 size_t rta_hybrid_workspace_bytes(const rta_hybrid_shape* shape, int batch) {
     if (check_shape(shape, batch)) return 0;
     size_t bytes = 0;
-    carve_work(shape, dims_of(shape, batch), nullptr, &bytes);
+    carve_work(shape, dims_of(shape, batch), nullptr, &bytes, true);
     return bytes;
 }
 
@@ -306,14 +318,15 @@ int rta_hybrid_decode_step_capture(const rta_hybrid_shape* shape, const rta_hybr
     if (!weights || !weights->layers || !weights->embed || !weights->lm_head || !weights->norm_final || !state ||
         !tokens || !workspace)
         return RTA_ERR_NULL;
-    if (workspace_bytes < rta_hybrid_workspace_bytes(shape, batch)) return RTA_ERR_WORKSPACE;
+    const Dims d = dims_of(shape, batch);
+    size_t need = 0;
+    Work w = carve_work(shape, d, workspace, &need, false);
+    if (workspace_bytes < need) return RTA_ERR_WORKSPACE;
     if (!host::aligned(state, 256) || !host::aligned(workspace, 256)) return RTA_ERR_ALIGN;
     if (capture && !(host::aligned(capture->residual, 4) && host::aligned(capture->kv, 4))) return RTA_ERR_ALIGN;
     if (capture && capture->residual && (capture->residual_from < 0 || capture->residual_from > shape->layers))
         return RTA_ERR_RANGE;
-    const Dims d = dims_of(shape, batch);
     const State st = carve_state(d, state, nullptr);
-    Work w = carve_work(shape, d, workspace, nullptr);
     int64_t embed_rb = 0;
     rc = host::embed_args(shape->fmt_embed, weights->embed, d.V, d.D, tokens, d.B, w.hidden, &embed_rb);
     if (rc) return rc;

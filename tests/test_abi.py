@@ -241,3 +241,24 @@ def test_workspaces_of_a_larger_batch_serve_every_smaller_one(lib):
         need = [query(b) for b in [*range(1, 140), 255, 256, 257, 300, 1000]]
         assert need[-1] > 0, name
         assert need == sorted(need), name
+
+
+def test_the_step_asks_for_no_more_than_its_own_batch_needs(lib):
+    """The size query of 65 sequences covers the 64 below it; a step of 65 itself takes the
+    smaller workspace of its own (24317440 bytes here), and not one byte less."""
+    from rta import model
+    T = _lib.TILED
+    hybrid = model._lib_h()
+    s = model.HybridShape(hidden=4096, layers=4, full_every=2, q_heads=4, kv_heads=2, head_dim=128, rec_heads=2,
+                          ff=12288, vocab=300, capacity=64, fmt_embed=_lib.Q4_K, fmt_proj=_lib.Q4_K | T,
+                          fmt_lm=_lib.Q6_K | T, fmt_k=_lib.Q4_K, fmt_v=_lib.Q6_K, rope_rotary=128, eps=1e-6,
+                          margin=1e-4, rope_theta=1e6)
+    w = model.HybridWeights(embed=FAKE.value, layers=ctypes.cast(FAKE.value, ctypes.POINTER(model.HybridLayer)),
+                            norm_final=FAKE.value, lm_head=FAKE.value)
+    own = 24317440
+    assert hybrid.rta_hybrid_workspace_bytes(ctypes.byref(s), 65) > own
+    # a misaligned state is refused (4) only after the workspace (5) was found large enough
+    step = lambda n: hybrid.rta_hybrid_decode_step(ctypes.byref(s), ctypes.byref(w), 65, FAKE_ODD, FAKE, None,  # noqa: E731
+                                                   FAKE, n, None)
+    assert step(own) == 4
+    assert step(own - 1) == 5
