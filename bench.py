@@ -826,8 +826,8 @@ WORKLOADS = {"gemv_q4k": w_gemv_q4k, "mlp": w_mlp, "lm_head": w_lm_head, "attent
 def main():
     args = parse()
     if args.gpus != 1:
-        print(json.dumps({"error": "this build measures one GPU; --gpus must be 1 (no multi-GPU path is "
-                                   "built: every GPU box here has one GPU)"}))
+        print(json.dumps({"error": "the benchmark measures one GPU; --gpus must be 1 (no multi-GPU path "
+                                   "is built)"}))
         sys.exit(2)
     import torch
     from rta import _lib
